@@ -219,6 +219,13 @@ NTOPS_API int ntops_cast(int src_dtype, int dst_dtype, int ndim, const int64_t* 
                const void* x, const int64_t* x_strides,
                void* y, const int64_t* y_strides, void* stream);
 
+/* y0 = x0, then y1 = x1: two copies of one shape and dtype (any of the
+ * dtypes), each tensor with its own strides, in one launch where neither
+ * copy touches what the other writes. */
+NTOPS_API int ntops_copy2(int dtype, int ndim, const int64_t* shape, const void* x0, const int64_t* x0_strides,
+               void* y0, const int64_t* y0_strides, const void* x1, const int64_t* x1_strides, void* y1,
+               const int64_t* y1_strides, void* stream);
+
 /* ---- row reductions --------------------------------------------------- */
 /* y[r, :] = x[r, :] * rsqrt(mean(x[r, :]^2) + eps) * w[r, :]   (fp32
  * accumulate, one rounding to dtype).  x and y are rows x cols with unit
@@ -323,6 +330,25 @@ NTOPS_API int ntops_sdpa(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t 
                const void* mask, int mask_dtype, const int64_t* mask_strides,
                int causal, double scale,
                void* out, const int64_t* out_strides, void* stream);
+
+/* ntops_sdpa with a caller-owned workspace of workspace_bytes device bytes
+ * (16-byte aligned), through which a few query rows over many keys (decode)
+ * spread the keys over the GPU: each slice of the keys writes fp32 partial
+ * results that a second kernel combines in slice order.  A missing or short
+ * workspace runs one block per key / value head; other problems ignore it. */
+NTOPS_API int ntops_sdpa_ws(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+               int64_t D, const void* q, const int64_t* q_strides,
+               const void* k, const int64_t* k_strides,
+               const void* v, const int64_t* v_strides,
+               const void* mask, int mask_dtype, const int64_t* mask_strides,
+               int causal, double scale,
+               void* out, const int64_t* out_strides,
+               void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Bytes of workspace ntops_sdpa_ws uses for this problem on the current
+ * device (0: it would not split the keys). */
+NTOPS_API int64_t ntops_sdpa_workspace(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+               int64_t D, int has_mask);
 
 /* ---- fused variants ------------------------------------------------------- */
 /* residual_out = x + residual (rounded to dtype) and y = rms_norm(residual_out)

@@ -66,6 +66,10 @@ _SIGNATURES = {
          _vp, _c_i64p, _vp],
     ),
     "ntops_cast": (_i, [_i, _i, _i, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp]),
+    "ntops_copy2": (
+        _i,
+        [_i, _i, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp],
+    ),
     "ntops_rms_norm": (_i, [_i, _i64, _i64, _vp, _i64, _vp, _i64, _i, _d, _vp, _i64, _vp]),
     "ntops_layer_norm": (_i, [_i, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _i, _d, _vp, _i64, _vp]),
     "ntops_softmax": (_i, [_i, _i, _i64, _i64, _i64, _vp, _c_i64p, _vp, _c_i64p, _vp]),
@@ -78,6 +82,12 @@ _SIGNATURES = {
         [_i, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _c_i64p,
          _i, _d, _vp, _c_i64p, _vp],
     ),
+    "ntops_sdpa_ws": (
+        _i,
+        [_i, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _c_i64p,
+         _i, _d, _vp, _c_i64p, _vp, _i64, _vp],
+    ),
+    "ntops_sdpa_workspace": (_i64, [_i, _i64, _i64, _i64, _i64, _i64, _i64, _i]),
     "ntops_add_rms_norm": (
         _i,
         [_i, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i, _d, _vp, _i64, _vp, _i64, _vp],

@@ -34,27 +34,10 @@
 //    of a head start first.
 // Generic path (fp32, other head dims up to 256, any strides): one wave per
 // query row, lanes split D, fp32 throughout.
-#include "mfma.h"
+#include "attention.h"
 
 namespace ntops {
 namespace {
-
-struct AttnArgs {
-  const void* q;
-  const void* k;
-  const void* v;
-  const void* mask;
-  void* o;
-  int64_t qs[4], ks[4], vs[4], ms[4], os[4];
-  int B, Hq, Hkv, Sq, Skv, D;
-  int mask_dtype;    // -1: none; NTOPS_BOOL (true = attend), NTOPS_F32 / F16 / BF16 (additive)
-  int causal;        // 0: none, 1: upper-left (kv <= q), 2: lower-right (kv <= q + Skv - Sq)
-  float scale_log2;  // scale * log2(e)
-};
-
-constexpr float kLog2e = 1.4426950408889634f;
-
-__device__ __forceinline__ float neg_inf() { return -__builtin_huge_valf(); }
 
 // Additive mask value at element offset `off`, in the base-2 domain.
 __device__ __forceinline__ float mask_log2(const AttnArgs& a, int64_t off) {
@@ -70,8 +53,6 @@ __device__ __forceinline__ float mask_log2(const AttnArgs& a, int64_t off) {
   }
 }
 
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
 // max(a, b, c) in one instruction, without the NaN-quieting moves the
 // compiler puts in front of fmaxf in IEEE mode (a NaN operand may be
 // dropped; a NaN score still reaches the output through its exponential).
@@ -79,16 +60,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
-}
-
-// Chunk slot of 16-byte chunk c of key row r in the V tile ([kv][d] with
-// D / 8 chunks per row), conflict-free for the transposing fragment reads.
-template <int D>
-__device__ __forceinline__ int vslot(int r, int c) {
-  if constexpr (D == 128)
-    return mnslot(r, c);
-  else
-    return c ^ (((r >> 1) & 1) << 2);
 }
 
 // B fragment of S = Q K^T: key rows n0 .. n0 + 31 (lane l: row n0 + (l & 31)),
@@ -1188,7 +1159,7 @@ int launch_flash_attn(const AttnArgs& a, hipStream_t st) {
 }
 
 template <typename T>
-int run_attention(const AttnArgs& a, hipStream_t st) {
+int run_attention(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st) {
   const auto unit_d = [&](const int64_t* s) { return s[3] == 1 && s[2] % 8 == 0 && s[1] % 8 == 0 && s[0] % 8 == 0; };
   // head dims up to 128 in multiples of 8 run on the D = 64 / 128 kernels,
   // the columns past the head dim zero in Q, K and V and dropped from O
@@ -1197,6 +1168,8 @@ int run_attention(const AttnArgs& a, hipStream_t st) {
                     a.os[1] % 4 == 0 && a.os[0] % 4 == 0 && aligned16(a.q) && aligned16(a.k) &&
                     aligned16(a.v) && (reinterpret_cast<uintptr_t>(a.o) & 7u) == 0;
   if constexpr (!std::is_same<T, float>::value) {
+    if (attn_decode_serves(a))
+      return attn_decode(std::is_same<T, __bf16>::value ? NTOPS_BF16 : NTOPS_F16, a, ws, ws_bytes, st);
     // DMA path: no explicit mask, a positive scale (the max of the scaled
     // scores is the scaled max), rows that do not overlap, and every key,
     // query and output row's byte offset (up to one block past the end)
@@ -1267,11 +1240,12 @@ int run_attention(const AttnArgs& a, hipStream_t st) {
 
 using namespace ntops;
 
-extern "C" int ntops_sdpa(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
-                          int64_t D, const void* q, const int64_t* q_strides, const void* k,
-                          const int64_t* k_strides, const void* v, const int64_t* v_strides,
-                          const void* mask, int mask_dtype, const int64_t* mask_strides, int causal,
-                          double scale, void* out, const int64_t* out_strides, void* stream) {
+extern "C" int ntops_sdpa_ws(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+                             int64_t D, const void* q, const int64_t* q_strides, const void* k,
+                             const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                             const void* mask, int mask_dtype, const int64_t* mask_strides, int causal,
+                             double scale, void* out, const int64_t* out_strides, void* workspace,
+                             int64_t workspace_bytes, void* stream) {
   if (B < 0 || Hq < 0 || Hkv < 0 || Sq < 0 || Skv < 0 || D < 0)
     return set_error(NTOPS_ERR_INVALID, "sdpa: negative size");
   if (B > 0x7fffffffLL || Hq > 0x7fffffffLL || Sq > 0x7fffffffLL || Skv > 0x7fffffffLL)
@@ -1314,6 +1288,23 @@ extern "C" int ntops_sdpa(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t
   hipStream_t st = static_cast<hipStream_t>(stream);
   return dispatch_float16_32(dtype, "sdpa", [&](auto tag) {
     using T = decltype(tag);
-    return run_attention<T>(a, st);
+    return run_attention<T>(a, workspace, workspace_bytes, st);
   });
+}
+
+extern "C" int ntops_sdpa(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+                          int64_t D, const void* q, const int64_t* q_strides, const void* k,
+                          const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                          const void* mask, int mask_dtype, const int64_t* mask_strides, int causal,
+                          double scale, void* out, const int64_t* out_strides, void* stream) {
+  return ntops_sdpa_ws(dtype, B, Hq, Hkv, Sq, Skv, D, q, q_strides, k, k_strides, v, v_strides, mask, mask_dtype,
+                       mask_strides, causal, scale, out, out_strides, nullptr, 0, stream);
+}
+
+extern "C" int64_t ntops_sdpa_workspace(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+                                        int64_t D, int has_mask) {
+  if ((dtype != NTOPS_BF16 && dtype != NTOPS_F16) || has_mask || B <= 0 || Hkv <= 0 || Hq <= 0 || Sq <= 0 || Skv <= 0 ||
+      D <= 0 || Hq % Hkv != 0 || Sq > 16 || B > 0x7fffffffLL || Hq > 0x7fffffffLL || Skv > 0x7fffffffLL)
+    return 0;
+  return attn_decode_workspace(B, Hq, Hkv, Sq, Skv, D);
 }

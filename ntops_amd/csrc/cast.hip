@@ -98,6 +98,50 @@ int launch_cast(int ndim, const int64_t* shape, const void* xv, const int64_t* x
   return check_launch("ntops_cast");
 }
 
+// Two strided copies of one shape and element type in one launch: grid row y
+// copies operand 2 y into operand 2 y + 1.  A decode step writes its key and
+// value rows into the cache this way; each copy is a few KiB, so what a
+// second launch costs (about 5 us) is most of the pair's time.
+template <typename E, typename I>
+__global__ __launch_bounds__(kThreads) void k_copy2_strided(KSpace<4, I> sp, const E* x0, E* y0, const E* x1, E* y1,
+                                                            I n) {
+  for (I i = static_cast<I>(blockIdx.x) * kThreads + threadIdx.x; i < n; i += static_cast<I>(gridDim.x) * kThreads) {
+    I off[4];
+    strided_offsets<4, I>(sp, i, off);
+    if (blockIdx.y == 0)
+      y0[off[1]] = x0[off[0]];
+    else
+      y1[off[3]] = x1[off[2]];
+  }
+}
+
+// Byte range [lo, hi) that the strided tensor at p touches.
+void touched(int ndim, const int64_t* shape, const void* p, const int64_t* st, int64_t size, uintptr_t* lo,
+             uintptr_t* hi) {
+  int64_t a = 0, b = 0;
+  for (int d = 0; d < ndim; ++d) {
+    const int64_t s = st[d] * (shape[d] - 1);
+    (s < 0 ? a : b) += s;
+  }
+  *lo = reinterpret_cast<uintptr_t>(p) + static_cast<uintptr_t>(a * size);
+  *hi = reinterpret_cast<uintptr_t>(p) + static_cast<uintptr_t>((b + 1) * size);
+}
+
+template <typename E>
+int launch_copy2(const StridedSpace<4>& sp, int64_t n, const void* x0, void* y0, const void* x1, void* y1,
+                 hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(ceil_div(n, kThreads), 65536)), 2);
+  if (fits_int32(sp, n + 65536 * static_cast<int64_t>(kThreads)))
+    hipLaunchKernelGGL((k_copy2_strided<E, int32_t>), grid, dim3(kThreads), 0, st, to_kspace<4, int32_t>(sp),
+                       static_cast<const E*>(x0), static_cast<E*>(y0), static_cast<const E*>(x1), static_cast<E*>(y1),
+                       static_cast<int32_t>(n));
+  else
+    hipLaunchKernelGGL((k_copy2_strided<E, int64_t>), grid, dim3(kThreads), 0, st, to_kspace<4, int64_t>(sp),
+                       static_cast<const E*>(x0), static_cast<E*>(y0), static_cast<const E*>(x1), static_cast<E*>(y1),
+                       n);
+  return check_launch("ntops_copy2");
+}
+
 }  // namespace
 }  // namespace ntops
 
@@ -122,4 +166,51 @@ extern "C" int ntops_cast(int src_dtype, int dst_dtype, int ndim, const int64_t*
       return launch_cast<S, D>(ndim, shape, x, x_strides, y, y_strides, st);
     });
   });
+}
+
+extern "C" int ntops_copy2(int dtype, int ndim, const int64_t* shape, const void* x0, const int64_t* x0_strides,
+                           void* y0, const int64_t* y0_strides, const void* x1, const int64_t* x1_strides, void* y1,
+                           const int64_t* y1_strides, void* stream) {
+  if (ndim < 0 || ndim > 64) return set_error(NTOPS_ERR_INVALID, "ntops_copy2: bad ndim %d", ndim);
+  const int64_t size = dtype_size(dtype);
+  if (size <= 0) return set_error(NTOPS_ERR_UNSUPPORTED, "ntops_copy2: unsupported dtype %d", dtype);
+  int64_t numel = 1;
+  for (int d = 0; d < ndim; ++d) {
+    if (shape[d] < 0) return set_error(NTOPS_ERR_INVALID, "ntops_copy2: negative extent");
+    numel *= shape[d];
+  }
+  if (numel == 0) return NTOPS_OK;
+  if (!x0 || !y0 || !x1 || !y1) return set_error(NTOPS_ERR_INVALID, "ntops_copy2: null pointer");
+  const int64_t* strides[4] = {x0_strides, y0_strides, x1_strides, y1_strides};
+  const void* ptr[4] = {x0, y0, x1, y1};
+  uintptr_t lo[4], hi[4];
+  for (int k = 0; k < 4; ++k) touched(ndim, shape, ptr[k], strides[k], size, &lo[k], &hi[k]);
+  // the second copy must see what the first wrote, and write after it
+  const auto meets = [&](int i, int j) { return lo[i] < hi[j] && lo[j] < hi[i]; };
+  StridedSpace<4> sp;
+  int64_t n = 0;
+  if (meets(1, 2) || meets(1, 3) || meets(0, 3) || !build_space<4>(ndim, shape, strides, &sp, &n)) {
+    const int rc = ntops_cast(dtype, dtype, ndim, shape, x0, x0_strides, y0, y0_strides, stream);
+    return rc != NTOPS_OK ? rc : ntops_cast(dtype, dtype, ndim, shape, x1, x1_strides, y1, y1_strides, stream);
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  // rows of whole 16-byte runs in every operand move as such runs
+  const int64_t v = 16 / size;
+  bool packs = sp.ndim > 0 && sp.shape[sp.ndim - 1] % v == 0;
+  for (int k = 0; k < 4; ++k) {
+    packs = packs && aligned16(ptr[k]) && sp.stride[k][sp.ndim - 1] == 1;
+    for (int d = 0; packs && d + 1 < sp.ndim; ++d) packs = sp.stride[k][d] % v == 0;
+  }
+  if (packs) {
+    sp.shape[sp.ndim - 1] /= v;
+    for (int k = 0; k < 4; ++k)
+      for (int d = 0; d + 1 < sp.ndim; ++d) sp.stride[k][d] /= v;
+    return launch_copy2<uint4>(sp, n / v, x0, y0, x1, y1, st);
+  }
+  switch (size) {
+    case 1: return launch_copy2<uint8_t>(sp, n, x0, y0, x1, y1, st);
+    case 2: return launch_copy2<uint16_t>(sp, n, x0, y0, x1, y1, st);
+    case 4: return launch_copy2<uint32_t>(sp, n, x0, y0, x1, y1, st);
+    default: return launch_copy2<uint64_t>(sp, n, x0, y0, x1, y1, st);
+  }
 }

@@ -22,6 +22,23 @@ from ntops_amd.torch.utils import _DeviceGuard, _cast_into, _strides, _to_dtype
 _MASK_DTYPES = (torch.bool, torch.float32, torch.float16, torch.bfloat16)
 
 
+def _write_slots(key, key_slot, value, value_slot):
+    """key_slot[...] = key and value_slot[...] = value; one launch for a pair
+    of plain copies (the usual case), else a cast kernel each."""
+    shape, dtype = key.shape, key.dtype
+    if all(t.shape == shape and t.dtype == dtype for t in (key_slot, value, value_slot)):
+        rc = _lib.load().ntops_copy2(
+            _lib.dtype_code(dtype), len(shape), _lib.i64_array(shape),
+            key.data_ptr(), _strides(key), key_slot.data_ptr(), _strides(key_slot),
+            value.data_ptr(), _strides(value), value_slot.data_ptr(), _strides(value_slot),
+            _lib.stream_of(value_slot),
+        )
+        _lib.check(rc, "ntops_amd.scaled_dot_product_attention")
+        return
+    _cast_into(key, key_slot)
+    _cast_into(value, value_slot)
+
+
 def scaled_dot_product_attention(
     query,
     key,
@@ -61,8 +78,7 @@ def scaled_dot_product_attention(
     if present_key is not None:
         # the reference's kernel assigns present_key_slot = present_key
         # (kernels/scaled_dot_product_attention.py:139-140) before attending
-        _cast_into(present_key, present_key_slot)
-        _cast_into(present_value, present_value_slot)
+        _write_slots(present_key, present_key_slot, present_value, present_value_slot)
 
     squeeze = query.dim() == 3
     if squeeze:
@@ -91,12 +107,20 @@ def scaled_dot_product_attention(
 
     output = torch.empty(query.shape[:-1] + (value.shape[-1],), dtype=value.dtype, device=dev)
     lib = _lib.load()
+    dt = _lib.dtype_code(query.dtype)
     with _DeviceGuard(dev):
-        rc = lib.ntops_sdpa(
-            _lib.dtype_code(query.dtype), B, Hq, key.shape[1], Sq, Skv, D,
+        # a few query rows over many keys spread the keys over the GPU through
+        # a workspace (fp32 partial results, combined in a fixed order)
+        ws, ws_bytes = None, 0
+        if Sq <= 16 and attn_mask is None:
+            ws_bytes = lib.ntops_sdpa_workspace(dt, B, Hq, key.shape[1], Sq, Skv, D, 0)
+            if ws_bytes > 0:
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        rc = lib.ntops_sdpa_ws(
+            dt, B, Hq, key.shape[1], Sq, Skv, D,
             query.data_ptr(), _strides(query), key.data_ptr(), _strides(key), value.data_ptr(), _strides(value),
             mask_ptr, mask_code, mask_strides, causal, float(scale),
-            output.data_ptr(), _strides(output), _lib.stream_of(output),
+            output.data_ptr(), _strides(output), None if ws is None else ws.data_ptr(), ws_bytes, _lib.stream_of(output),
         )
     _lib.check(rc, "ntops_amd.scaled_dot_product_attention")
     return output.squeeze(0) if squeeze else output
