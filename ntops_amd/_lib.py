@@ -146,7 +146,23 @@ def load():
             fn.restype = res
             fn.argtypes = args
         _lib = lib
+        _init_fast(lib)
     return _lib
+
+
+try:
+    # the wrappers' native host path (csrc/host/fast.cpp); without it they take
+    # the Python path to the same kernels
+    from ntops_amd import _fast as fast
+except ImportError:
+    fast = None
+
+
+def _init_fast(lib):
+    """Hands the native host path the loaded library's entry points."""
+    if fast is not None and _raw_stream is not None:
+        addresses = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _SIGNATURES}
+        fast.init(addresses, getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device), _raw_stream)
 
 
 def i64_array(values):

@@ -18,7 +18,14 @@ from ntops_amd import _lib
 from ntops_amd.torch.utils import _DeviceGuard, _norm_param, _rows_of
 
 
+_EPS = torch.finfo(torch.float32).eps
+
+
 def add_rms_norm(input, residual, normalized_shape, weight=None, eps=None, *, inplace=False):
+    if _lib.fast is not None and not inplace:
+        r = _lib.fast.add_rms_norm(input, residual, normalized_shape, weight, _EPS if eps is None else eps)
+        if r is not None:
+            return r
     if isinstance(normalized_shape, int):
         normalized_shape = (normalized_shape,)
     normalized_shape = tuple(normalized_shape)

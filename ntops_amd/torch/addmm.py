@@ -5,10 +5,15 @@ beta == 0 ignores `input` entirely, as torch does."""
 
 import torch
 
+from ntops_amd import _lib
 from ntops_amd.torch._gemm import gemm
 
 
 def addmm(input, mat1, mat2, *, beta=1, alpha=1, out=None):
+    if _lib.fast is not None and out is None:
+        r = _lib.fast.addmm(input, mat1, mat2, beta, alpha)
+        if r is not None:
+            return r
     if mat1.dim() != 2 or mat2.dim() != 2:
         raise RuntimeError("addmm: expected 2-D matrices")
     m, k = mat1.shape

@@ -10,6 +10,10 @@ from ntops_amd.torch.utils import _DeviceGuard, _norm_param, _rows_of
 
 
 def layer_norm(input, normalized_shape, weight=None, bias=None, eps=1e-5):
+    if _lib.fast is not None:
+        r = _lib.fast.layer_norm(input, normalized_shape, weight, bias, eps)
+        if r is not None:
+            return r
     if isinstance(normalized_shape, int):
         normalized_shape = (normalized_shape,)
 

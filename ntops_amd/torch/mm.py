@@ -2,10 +2,15 @@
 
 import torch
 
+from ntops_amd import _lib
 from ntops_amd.torch._gemm import gemm
 
 
 def mm(input, mat2, *, out=None):
+    if _lib.fast is not None and out is None:
+        r = _lib.fast.mm(input, mat2)
+        if r is not None:
+            return r
     if input.dim() != 2 or mat2.dim() != 2:
         raise RuntimeError("mm: expected 2-D tensors")
     m, k = input.shape

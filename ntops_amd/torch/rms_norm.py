@@ -17,7 +17,14 @@ from ntops_amd import _lib
 from ntops_amd.torch.utils import _DeviceGuard, _norm_param, _rows_of
 
 
+_EPS = torch.finfo(torch.float32).eps
+
+
 def rms_norm(input, normalized_shape, weight=None, eps=None):
+    if _lib.fast is not None:
+        r = _lib.fast.rms_norm(input, normalized_shape, weight, _EPS if eps is None else eps)
+        if r is not None:
+            return r
     if isinstance(normalized_shape, int):
         normalized_shape = (normalized_shape,)
 

@@ -15,6 +15,10 @@ from ntops_amd.torch.utils import _DeviceGuard, _contiguous, _to_dtype
 
 
 def rotary_position_embedding_qk(q, k, sin_table, cos_table, interleaved=True, inplace=False):
+    if _lib.fast is not None and not inplace:
+        r = _lib.fast.rope_qk(q, k, sin_table, cos_table, interleaved)
+        if r is not None:
+            return r
     if q.dim() != 4 or k.dim() != 4:
         raise RuntimeError("rotary_position_embedding_qk: q and k must be (batch, seq, heads, dim)")
     batch_size, seq_len, q_heads, emb_dim = q.shape

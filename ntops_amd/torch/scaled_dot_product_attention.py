@@ -57,6 +57,15 @@ def scaled_dot_product_attention(
     assert dropout_p == 0, "`dropout_p` is not supported yet."
     assert attn_mask is None or not is_causal, "Cannot use `attn_mask` and `is_causal` together."
 
+    if _lib.fast is not None:
+        causal = 0
+        if is_causal:
+            causal = int(CausalVariant.UPPER_LEFT if causal_variant is None else CausalVariant(causal_variant))
+        r = _lib.fast.sdpa(query, key, value, attn_mask, causal, scale, enable_gqa, present_key, present_value,
+                           present_key_slot, present_value_slot)
+        if r is not None:
+            return r
+
     num_heads_q, num_heads_kv = query.shape[-3], key.shape[-3]
     assert num_heads_kv == value.shape[-3], "Number of heads in `key` and `value` must be the same."
     if not enable_gqa:

@@ -7,6 +7,10 @@ from ntops_amd.torch.utils import _unary
 
 
 def silu(input, inplace=False):
+    if _lib.fast is not None and not inplace:
+        r = _lib.fast.unary(_lib.UNARY_SILU, input)
+        if r is not None:
+            return r
     if not input.dtype.is_floating_point:
         raise RuntimeError(f'"silu" not implemented for {input.dtype}')
 

@@ -36,6 +36,10 @@ def _view_strides(input, dim):
 
 
 def softmax(input, dim, dtype=None):
+    if _lib.fast is not None and dtype is None:
+        r = _lib.fast.softmax(input, dim)
+        if r is not None:
+            return r
     tensor_dtype = dtype if dtype is not None else input.dtype
     if tensor_dtype not in (torch.float32, torch.float16, torch.bfloat16, torch.float64):
         raise RuntimeError(f"softmax: unsupported output dtype {tensor_dtype}")
