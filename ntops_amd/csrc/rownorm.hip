@@ -493,10 +493,9 @@ __global__ __launch_bounds__(kWideThreads) void k_ln_wide(const T* __restrict__ 
 // kernels (register-resident, one HBM read and one write); lanes 0..head-1
 // of the row's first wave hold the head elements and lanes 0..tail-1 of its
 // last wave the tail (element loads and stores through buffer resources
-// whose extent is the head / tail: branch-free, zeros elsewhere).  The
-// weight and bias rows are staged once per block in LDS, where element j is
-// read at any offset: a pack of the row starts `head` elements past a
-// parameter pack boundary.
+// whose extent is the head / tail: branch-free, zeros elsewhere).  A pack of
+// the row starts `head` elements past a parameter pack boundary, so weight
+// and bias are loaded at any element's address (OddParam).
 struct OddRow {
   int head, npk, tail;
 };
@@ -568,49 +567,99 @@ __device__ __forceinline__ float odd_sumsq(const OddSlot<T, CHUNKS>& d) {
   return fmaf(to_f(d.tl), to_f(d.tl), ss);
 }
 
-// Stages `cols` parameters of type W at `src` into LDS at `dst` (16-byte
-// packs, then the last cols % per-pack elements one by one).
-template <typename W>
-__device__ __forceinline__ void stage_param(W* dst, const W* src, int cols) {
-  constexpr int kPer = Pack16<W>::N;
-  const int full = cols / kPer;
-  for (int q = threadIdx.x; q < full; q += blockDim.x)
-    *reinterpret_cast<u32x4*>(dst + q * kPer) = *reinterpret_cast<const u32x4*>(src + q * kPer);
-  for (int e = full * kPer + threadIdx.x; e < cols; e += blockDim.x) dst[e] = src[e];
-}
+// The weight (or bias) values of the elements a lane holds of a row: a pack of
+// the row starts `head` elements past a pack of the parameters, so they are
+// loaded by 16-byte loads at any element's address, straight from cache: up
+// to 16 VGPRs of them with the row, more at their use.  (Staged in LDS per
+// row and read back one element at a time, layer_norm on bf16 (16384, 4100)
+// took 69.3 us, 51.8 this way.)  A null parameter reads as `none`.
+template <typename T, typename W, int CHUNKS, int WPR>
+struct OddParam {
+  static constexpr int V = Pack16<T>::N, kPer = Pack16<W>::N;
+  static constexpr bool kEarly = CHUNKS * V * sizeof(W) <= 64;
+  static constexpr uint32_t kPast = 0x80000000u;  // past every extent: reads as zero
+  struct Chunk {
+    W v[V];
+  };
+  Chunk early[kEarly ? CHUNKS : 1];
+  W hd, tl;
+  __amdgpu_buffer_rsrc_t r;
+  bool any;
+  float none;
 
-// Writes one row's normalised values: packs, head and tail; f(v, j) gives
-// the output for element value v at column j.
-template <int WPR, typename T, int CHUNKS, typename F>
+  __device__ __forceinline__ Chunk load(const OddRow& g, const RowPos& p, int c) const {
+    const int pk = pack_of<WPR>(p, c);
+    const uint32_t at = pk < g.npk ? static_cast<uint32_t>((g.head + pk * V) * sizeof(W)) : kPast;
+    Chunk o;
+#pragma unroll
+    for (int q = 0; q < V / kPer; ++q) {
+      const Pack16<W> w = __builtin_bit_cast(Pack16<W>, __builtin_amdgcn_raw_buffer_load_b128(r, at, q * 16, 0));
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) o.v[q * kPer + i] = w.v[i];
+    }
+    return o;
+  }
+  __device__ __forceinline__ W elem(bool own, int j) const {
+    const uint32_t at = own ? static_cast<uint32_t>(j * sizeof(W)) : kPast;
+    if constexpr (sizeof(W) == 2)
+      return __builtin_bit_cast(W, __builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0));
+    else
+      return __builtin_bit_cast(W, __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
+  }
+  __device__ __forceinline__ void init(const W* src, float without, int cols, const OddRow& g, const RowPos& p,
+                                       const OddSlot<T, CHUNKS>& d) {
+    any = src != nullptr;
+    none = without;
+    r = buffer_rsrc(src, any ? static_cast<uint32_t>(cols * sizeof(W)) : 0u);
+    if constexpr (kEarly) {
+#pragma unroll
+      for (int c = 0; c < CHUNKS; ++c) early[c] = load(g, p, c);
+    }
+    hd = elem(d.own_hd, p.lane);
+    tl = elem(d.own_tl, g.head + g.npk * V + p.lane);
+  }
+  __device__ __forceinline__ Chunk chunk(const OddRow& g, const RowPos& p, int c) const {
+    if constexpr (kEarly)
+      return early[c];
+    else
+      return load(g, p, c);
+  }
+  __device__ __forceinline__ float value(W w) const { return any ? static_cast<float>(w) : none; }
+};
+
+// Writes one row: packs, head and tail; f(v, w, b) gives the output of element
+// value v under the parameter values w and b.
+template <int WPR, typename T, int CHUNKS, typename PW, typename PB, typename F>
 __device__ __forceinline__ void odd_store(T* row, const OddRow& g, bool row_ok, const RowPos& p,
-                                          const OddSlot<T, CHUNKS>& d, F f) {
+                                          const OddSlot<T, CHUNKS>& d, const PW& w, const PB& b, F f) {
   constexpr int V = Pack16<T>::N;
   const bool first = p.wave_in_row == 0, last = p.wave_in_row == WPR - 1;
   const __amdgpu_buffer_rsrc_t rp = buffer_rsrc(row + g.head, row_ok ? g.npk * 16u : 0u);
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
-    const int pk = pack_of<WPR>(p, c);
-    const int j0 = g.head + pk * V;
+    const auto wc = w.chunk(g, p, c);
+    const auto bc = b.chunk(g, p, c);
     Pack16<T> o;
 #pragma unroll
-    for (int i = 0; i < V; ++i) o.v[i] = f(d.pk[c].v[i], pk < g.npk ? j0 + i : 0);
-    buffer_store16_nt(rp, pk * 16u, o);
+    for (int i = 0; i < V; ++i) o.v[i] = f(d.pk[c].v[i], w.value(wc.v[i]), b.value(bc.v[i]));
+    buffer_store16_nt(rp, pack_of<WPR>(p, c) * 16u, o);
   }
   const __amdgpu_buffer_rsrc_t rh = buffer_rsrc(row, row_ok && first ? g.head * sizeof(T) : 0u);
   const __amdgpu_buffer_rsrc_t rt =
       buffer_rsrc(row + g.head + g.npk * V, row_ok && last ? g.tail * sizeof(T) : 0u);
-  buffer_store_elem<T>(rh, p.lane * sizeof(T), f(d.hd, d.own_hd ? p.lane : 0));
-  buffer_store_elem<T>(rt, p.lane * sizeof(T), f(d.tl, d.own_tl ? g.head + g.npk * V + p.lane : 0));
+  buffer_store_elem<T>(rh, p.lane * sizeof(T), f(d.hd, w.value(w.hd), b.value(b.hd)));
+  buffer_store_elem<T>(rt, p.lane * sizeof(T), f(d.tl, w.value(w.tl), b.value(b.tl)));
 }
-
-// Bytes of LDS the odd-layout kernels stage per parameter row.
-template <typename W>
-__host__ __device__ inline int64_t odd_param_bytes(int64_t cols) {
-  return (cols * static_cast<int64_t>(sizeof(W)) + 15) / 16 * 16;
-}
-// Their most staged-parameter LDS: under the 64 KiB a launch may take without
-// raising its limit, with room for the kernels' static reduction scratch.
-constexpr int64_t kOddLdsMax = 60 * 1024;
+// No parameter at all.
+template <typename T>
+struct OddNone {
+  struct Chunk {
+    T v[Pack16<T>::N];
+  };
+  T hd, tl;
+  __device__ __forceinline__ Chunk chunk(const OddRow&, const RowPos&, int) const { return Chunk{}; }
+  __device__ __forceinline__ float value(T) const { return 0.f; }
+};
 
 template <typename T, typename W, int CHUNKS, int WPR>
 __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_rms_odd(
@@ -618,8 +667,6 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_rms_odd(
     int64_t rows, int cols, float eps) {
   constexpr int RPB = RowShape<WPR>::kRowsPerBlock;
   __shared__ float red[RPB * WPR];
-  extern __shared__ __attribute__((aligned(16))) char psm[];
-  W* wl = reinterpret_cast<W*>(psm);
   const RowPos p = row_pos<WPR>();
   const int64_t row = block_id() * RPB + p.row_in_block;
   const bool row_ok = row < rows;
@@ -627,13 +674,12 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_rms_odd(
   const OddRow g = odd_row(xr, cols);
   OddSlot<T, CHUNKS> d;
   odd_load<WPR>(d, xr, g, row_ok, p);
-  if (w != nullptr) stage_param(wl, w, cols);
+  OddParam<T, W, CHUNKS, WPR> pw;
+  pw.init(w, 1.0f, cols, g, p, d);
   float ss[1] = {odd_sumsq(d)};
-  __syncthreads();  // the staged weight (and, for one wave per row, nothing else)
   rows_sum<WPR>(ss, red, p);
   const float rstd = 1.0f / __fsqrt_rn(ss[0] / static_cast<float>(cols) + eps);
-  odd_store<WPR>(y + (row_ok ? row : 0) * ys, g, row_ok, p, d, [&](T v, int j) {
-    const float wv = w != nullptr ? static_cast<float>(wl[j]) : 1.0f;
+  odd_store<WPR>(y + (row_ok ? row : 0) * ys, g, row_ok, p, d, pw, OddNone<T>{}, [&](T v, float wv, float) {
     return static_cast<T>(mul_nc(mul_nc(to_f(v), rstd), wv));
   });
 }
@@ -648,8 +694,6 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_add_rms_odd(
   constexpr int V = Pack16<T>::N;
   constexpr int RPB = RowShape<WPR>::kRowsPerBlock;
   __shared__ float red[RPB * WPR];
-  extern __shared__ __attribute__((aligned(16))) char psm[];
-  W* wl = reinterpret_cast<W*>(psm);
   const RowPos p = row_pos<WPR>();
   const int64_t row = block_id() * RPB + p.row_in_block;
   const bool row_ok = row < rows;
@@ -658,7 +702,8 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_add_rms_odd(
   OddSlot<T, CHUNKS> d, e;
   odd_load<WPR>(d, x + rc * xs, g, row_ok, p);
   odd_load<WPR>(e, res + rc * rs, g, row_ok, p);
-  if (w != nullptr) stage_param(wl, w, cols);
+  OddParam<T, W, CHUNKS, WPR> pw;
+  pw.init(w, 1.0f, cols, g, p, d);
   auto add = [](T a, T b) { return static_cast<T>(add_nc(to_f(a), to_f(b))); };
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c)
@@ -666,13 +711,11 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_add_rms_odd(
     for (int i = 0; i < V; ++i) d.pk[c].v[i] = add(d.pk[c].v[i], e.pk[c].v[i]);
   d.hd = add(d.hd, e.hd);
   d.tl = add(d.tl, e.tl);
-  odd_store<WPR>(ro + rc * ros, g, row_ok, p, d, [](T v, int) { return v; });
+  odd_store<WPR>(ro + rc * ros, g, row_ok, p, d, OddNone<T>{}, OddNone<T>{}, [](T v, float, float) { return v; });
   float ss[1] = {odd_sumsq(d)};
-  __syncthreads();
   rows_sum<WPR>(ss, red, p);
   const float rstd = 1.0f / __fsqrt_rn(ss[0] / static_cast<float>(cols) + eps);
-  odd_store<WPR>(y + rc * ys, g, row_ok, p, d, [&](T v, int j) {
-    const float wv = w != nullptr ? static_cast<float>(wl[j]) : 1.0f;
+  odd_store<WPR>(y + rc * ys, g, row_ok, p, d, pw, OddNone<T>{}, [&](T v, float wv, float) {
     return static_cast<T>(mul_nc(mul_nc(to_f(v), rstd), wv));
   });
 }
@@ -685,9 +728,6 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_ln_odd(
   constexpr int RPB = RowShape<WPR>::kRowsPerBlock;
   __shared__ float red0[RPB * WPR];
   __shared__ float red1[RPB * WPR];
-  extern __shared__ __attribute__((aligned(16))) char psm[];
-  W* wl = reinterpret_cast<W*>(psm);
-  W* bl = reinterpret_cast<W*>(psm + odd_param_bytes<W>(cols));
   const RowPos p = row_pos<WPR>();
   const int64_t row = block_id() * RPB + p.row_in_block;
   const bool row_ok = row < rows;
@@ -695,8 +735,9 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_ln_odd(
   const OddRow g = odd_row(xr, cols);
   OddSlot<T, CHUNKS> d;
   odd_load<WPR>(d, xr, g, row_ok, p);
-  if (w != nullptr) stage_param(wl, w, cols);
-  if (b != nullptr) stage_param(bl, b, cols);
+  OddParam<T, W, CHUNKS, WPR> pw, pb;
+  pw.init(w, 1.0f, cols, g, p, d);
+  pb.init(b, 0.0f, cols, g, p, d);
   float acc[1];
   {
     float s0 = to_f(d.hd), s1 = 0.f;
@@ -709,7 +750,6 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_ln_odd(
       }
     acc[0] = s0 + s1 + to_f(d.tl);
   }
-  __syncthreads();
   rows_sum<WPR>(acc, red0, p);
   const float mean = acc[0] / static_cast<float>(cols);
   {
@@ -732,9 +772,7 @@ __global__ __launch_bounds__(RowShape<WPR>::kThreads) void k_ln_odd(
   const float var = acc[0] * (1.0f / static_cast<float>(cols));
   const float rstd = 1.0f / __fsqrt_rn(fmaxf(var, 0.f) + eps);
   const float shift = -rstd * mean;
-  odd_store<WPR>(y + (row_ok ? row : 0) * ys, g, row_ok, p, d, [&](T v, int j) {
-    const float wv = w != nullptr ? static_cast<float>(wl[j]) : 1.0f;
-    const float bv = b != nullptr ? static_cast<float>(bl[j]) : 0.0f;
+  odd_store<WPR>(y + (row_ok ? row : 0) * ys, g, row_ok, p, d, pw, pb, [&](T v, float wv, float bv) {
     return static_cast<T>(fmaf(fmaf(to_f(v), rstd, shift), wv, bv));
   });
 }
@@ -791,13 +829,12 @@ int run_rms(int64_t rows, int64_t cols, const void* xv, int64_t xs, const void* 
                        w, y, ys, rows, static_cast<int>(cols), feps);
     return check_launch("rms_norm");
   }
-  const int64_t lds = w != nullptr ? odd_param_bytes<W>(cols) : 0;
-  if (same_layout<T>(x, xs, y, ys) && (w == nullptr || (aligned16(w) && wrs == 0)) && lds <= kOddLdsMax &&
+  if (same_layout<T>(x, xs, y, ys) && (w == nullptr || (aligned16(w) && wrs == 0)) &&
       pick_odd_cfg(cols, V, &cfg)) {
 #define NTOPS_RMS_ODD_CASE(CH, WP)                                                                \
   if (cfg.chunks == CH && cfg.wpr == WP) {                                                        \
     hipLaunchKernelGGL((k_rms_odd<T, W, CH, WP>), blocks_2d(ceil_div(rows, RowShape<WP>::kRowsPerBlock)), \
-                       dim3(RowShape<WP>::kThreads), static_cast<unsigned>(lds), st, x, xs, w, y, ys,    \
+                       dim3(RowShape<WP>::kThreads), 0, st, x, xs, w, y, ys,    \
                        rows, static_cast<int>(cols), feps);                                       \
     return check_launch("rms_norm");                                                              \
   }
@@ -843,13 +880,12 @@ int run_ln(int64_t rows, int64_t cols, const void* xv, int64_t xs, const void* w
                        b, y, ys, rows, static_cast<int>(cols), feps);
     return check_launch("layer_norm");
   }
-  const int64_t lds = (w != nullptr || b != nullptr) ? 2 * odd_param_bytes<W>(cols) : 0;
   if (same_layout<T>(x, xs, y, ys) && (w == nullptr || aligned16(w)) && (b == nullptr || aligned16(b)) &&
-      wrs == 0 && lds <= kOddLdsMax && pick_odd_cfg(cols, V, &cfg)) {
+      wrs == 0 && pick_odd_cfg(cols, V, &cfg)) {
 #define NTOPS_LN_ODD_CASE(CH, WP)                                                                 \
   if (cfg.chunks == CH && cfg.wpr == WP) {                                                        \
     hipLaunchKernelGGL((k_ln_odd<T, W, CH, WP>), blocks_2d(ceil_div(rows, RowShape<WP>::kRowsPerBlock)), \
-                       dim3(RowShape<WP>::kThreads), static_cast<unsigned>(lds), st, x, xs, w, b, y, ys, \
+                       dim3(RowShape<WP>::kThreads), 0, st, x, xs, w, b, y, ys, \
                        rows, static_cast<int>(cols), feps);                                       \
     return check_launch("layer_norm");                                                            \
   }
@@ -891,13 +927,12 @@ int run_add_rms(int64_t rows, int64_t cols, const void* xv, int64_t xs, const vo
     NTOPS_ROW_CASES(NTOPS_ADD_RMS_CASE)
 #undef NTOPS_ADD_RMS_CASE
   }
-  const int64_t lds = w != nullptr ? odd_param_bytes<W>(cols) : 0;
   if (same_layout<T>(x, xs, y, ys) && same_layout<T>(r, rs, y, ys) && same_layout<T>(ro, ros, y, ys) &&
-      (w == nullptr || (aligned16(w) && wrs == 0)) && lds <= kOddLdsMax && pick_odd_cfg(cols, V, &cfg)) {
+      (w == nullptr || (aligned16(w) && wrs == 0)) && pick_odd_cfg(cols, V, &cfg)) {
 #define NTOPS_ADD_RMS_ODD_CASE(CH, WP)                                                            \
   if (cfg.chunks == CH && cfg.wpr == WP) {                                                        \
     hipLaunchKernelGGL((k_add_rms_odd<T, W, CH, WP>), blocks_2d(ceil_div(rows, RowShape<WP>::kRowsPerBlock)), \
-                       dim3(RowShape<WP>::kThreads), static_cast<unsigned>(lds), st, x, xs, r, rs, w, y, ys,   \
+                       dim3(RowShape<WP>::kThreads), 0, st, x, xs, r, rs, w, y, ys,   \
                        ro, ros, rows, static_cast<int>(cols), feps);                              \
     return check_launch("add_rms_norm");                                                          \
   }
