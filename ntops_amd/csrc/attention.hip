@@ -62,6 +62,22 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
+// Max of a lane's 32 scores of a tile: 16 three-way maxima in a tree.
+__device__ __forceinline__ float max32(const f32x16 (&s)[2]) {
+  float v[32];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[16 * u + e] = s[u][e];
+  float m1[11];
+#pragma unroll
+  for (int i = 0; i < 10; ++i) m1[i] = max3(v[3 * i], v[3 * i + 1], v[3 * i + 2]);
+  m1[10] = max3(v[30], v[31], v[31]);
+  const float m2a = max3(m1[0], m1[1], m1[2]), m2b = max3(m1[3], m1[4], m1[5]);
+  const float m2c = max3(m1[6], m1[7], m1[8]), m2d = max3(m1[9], m1[10], m1[10]);
+  return max3(m2a, m2b, max3(m2c, m2d, m2d));
+}
+
 // B fragment of S = Q K^T: key rows n0 .. n0 + 31 (lane l: row n0 + (l & 31)),
 // d = 16 ks + 8 (l >> 5) .. + 7.
 template <int D>
@@ -169,8 +185,8 @@ struct KvDma {
   }
 };
 
-// MM: explicit-mask mode -- 0 none, 1 runs of 4 keys per access (rows
-// 4-element aligned), 2 element loads; ESZ: mask element bytes (1 bool, 2
+// MM: explicit-mask mode -- 0 none, 1 / 2 the last, partial tile by runs of 4
+// keys (rows 4-element aligned) / by elements; ESZ: mask element bytes (1 bool, 2
 // fp16 / bf16, 4 fp32).  Both are template parameters so that every mask
 // load writes fixed registers.
 template <typename T, int D, int MM, int ESZ>
@@ -208,6 +224,13 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     else
       qf[ks] = u32x4{0, 0, 0, 0};
   }
+  // a negative scale: -Q under its magnitude, so that the max of the scaled
+  // scores is the scaled max (a zero scale takes the generic kernel)
+  const bool neg = a.scale_log2 < 0.f;
+  if (neg) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] ^= 0x80008000u;
+  }
 
   int kv_end = a.Skv;
   if (a.causal) kv_end = max(0, min(a.Skv, q0 + BM + off));
@@ -218,9 +241,13 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
   // S * scale carries it; its raw data for tile j + 1 is loaded while tile j
   // is softmaxed and multiplied by V (S's registers are free then), through
   // a buffer resource over this (batch, head)'s plane (a row past Sq or a key
-  // past the plane reads 0; such keys are masked anyway).  mmode 1: every run
-  // of 4 keys of a lane is one access (rows 4-element aligned); 2: element
-  // loads.
+  // past the plane reads 0; such keys are masked anyway).  Tiles that the mask
+  // leaves open start from zero.  What this kernel's masked time was before
+  // the wide loads, the open tiles and the fused softmax (one fma per score,
+  // three-way maxima, O rescaled only past 2^8), (8, 16, 1000, 64) f16 bool:
+  // 118 us -> 79 with the softmax and open tiles -> 62 with the wide loads
+  // (float 102 -> 63; (4, 32, 2048, 128) bf16 bool 607 -> 324; rows of 1397
+  // keys, read element by element before, 159 -> 71).
   constexpr int esz = ESZ;
   constexpr int mmode = MM;
   const char* mp = mmode != 0 ? static_cast<const char*>(a.mask) + (b * a.ms[0] + h * a.ms[1]) * esz
@@ -229,19 +256,48 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       mmode != 0 ? (static_cast<int64_t>(a.Sq - 1) * a.ms[2] + static_cast<int64_t>(a.Skv - 1) + 1) * esz : 0;
   const __amdgpu_buffer_rsrc_t rm = buffer_rsrc(mp, static_cast<uint32_t>(mext));
   const int64_t mrow = static_cast<int64_t>(my_q) * a.ms[2];
-  const float inv_scale = kLog2e / a.scale_log2;
+  const float inv_scale = kLog2e / (neg ? -a.scale_log2 : a.scale_log2);
   // raw mask data, run r (keys kv .. kv + 3 of mask_issue) in mraw[4 r ..]:
   // one word (bool runs), two (16-bit runs), four (fp32 runs or elementwise
   // loads) -- the same slots in every mode, so that the compiler, which
   // merges the branches' stores, never sees a variable index
   uint32_t mraw[32];
+  // A tile that ends inside the rows (kWide): a lane loads 32 consecutive keys
+  // of its row by 16-byte accesses -- its half lane ^ 32 the other 32 -- and
+  // mask_swap deals the runs of 4 out when they have landed: 2 (bool) or 4
+  // (16-bit) instructions that touch 64 row pieces each instead of 8.  The
+  // last tile loads run by run, nothing past the rows' last key.
+  // Rows may start anywhere.  (fp32: 8 runs of 16 bytes either way.)
+  constexpr bool kWide = mmode != 0 && esz <= 2;
+  auto tile_in = [&](int j) { return (j + 1) * BN <= a.Skv; };
   auto mask_issue = [&](int j) {
     const bool row_ok = my_q < a.Sq;
+    if constexpr (kWide) {
+      if (tile_in(j)) {
+        const uint32_t o = row_ok ? static_cast<uint32_t>((mrow + j * BN + 32 * (lane >> 5)) * esz) : kOOB;
+#pragma unroll
+        for (int k = 0; k < 2 * esz; ++k) {
+          const u32x4 w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rm, o, k * 16, 0));
+          if constexpr (esz == 1) {
+            mraw[8 * k] = w.x;
+            mraw[8 * k + 16] = w.y;
+            mraw[8 * k + 4] = w.z;
+            mraw[8 * k + 20] = w.w;
+          } else {
+            mraw[4 * k] = w.x;
+            mraw[4 * k + 1] = w.y;
+            mraw[4 * k + 16] = w.z;
+            mraw[4 * k + 17] = w.w;
+          }
+        }
+        return;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < 8; ++r) {  // run r: keys kv .. kv + 3
       const int kv = j * BN + 32 * (r >> 2) + 8 * (r & 3) + 4 * (lane >> 5);
       const uint32_t o = row_ok && kv < a.Skv ? static_cast<uint32_t>((mrow + kv) * esz) : kOOB;
-      if constexpr (mmode == 1) {
+      if (mmode == 1 || (esz == 4 && tile_in(j))) {
         if constexpr (esz == 1) {
           mraw[4 * r] = __builtin_amdgcn_raw_buffer_load_b32(rm, o, 0, 0);
         } else if constexpr (esz == 2) {
@@ -266,17 +322,67 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       }
     }
   };
+  // The landed tile j as packed runs of 4 in mraw[4 r ..].  Wide: even runs to
+  // lanes 0-31, odd ones to lanes 32-63 -- the low half of one register trades
+  // places with the high half of the other.
+  auto mask_pack = [&](int j) {
+    if constexpr (kWide) {
+      if (tile_in(j)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int w = 0; w < esz; ++w) {
+            const auto r = __builtin_amdgcn_permlane32_swap(mraw[4 * i + w], mraw[16 + 4 * i + w], false, false);
+            mraw[4 * i + w] = r[0];
+            mraw[16 + 4 * i + w] = r[1];
+          }
+      } else if constexpr (mmode == 2) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          uint32_t* m = &mraw[4 * r];
+          if constexpr (esz == 1) {
+            m[0] = m[0] | m[1] << 8 | m[2] << 16 | m[3] << 24;
+          } else {
+            m[0] = m[0] | m[1] << 16;
+            m[1] = m[2] | m[3] << 16;
+          }
+        }
+      }
+    }
+  };
+  // True when the mask leaves every score of the wave's tile as it is (all
+  // true, or all +0): most tiles of a padding or causal mask, whose S then
+  // starts at zero instead of 32 selects or conversions.
+  auto mask_open = [&]() {
+    constexpr int kPer = esz;  // words of a run
+    uint32_t a_ = ~0u, o_ = 0u;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        if constexpr (esz == 1) a_ &= mraw[4 * r + i];
+        o_ |= mraw[4 * r + i];
+      }
+    if constexpr (esz == 1) {
+      return __all(a_ == 0x01010101u && o_ == 0x01010101u);
+    } else {
+      return __all(o_ == 0u);
+    }
+  };
   // S's initial value: mask / scale (bool: 0 or -inf) for element 4 q + e of half t
   auto mask_init = [&](f32x16 (&sv)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sv[t][e] = 0.f;
+    if (mask_open()) return;
 #pragma unroll
     for (int r = 0; r < 8; ++r)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        uint32_t w;
-        if constexpr (mmode == 1)
-          w = esz == 1 ? (mraw[4 * r] >> (8 * e)) : esz == 2 ? (mraw[4 * r + (e >> 1)] >> (16 * (e & 1))) : mraw[4 * r + e];
-        else
-          w = mraw[4 * r + e];
+        const uint32_t w = esz == 1   ? (mraw[4 * r] >> (8 * e))
+                           : esz == 2 ? (mraw[4 * r + (e >> 1)] >> (16 * (e & 1)))
+                                      : mraw[4 * r + e];
         float m;
         if constexpr (esz == 1)
           m = (w & 0xffu) ? 0.f : neg_inf();
@@ -308,7 +414,12 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
-  float m_i = neg_inf(), l_i = 0.f;  // running max (base 2) and sum of row my_q
+  float m_i = neg_inf(), l_i = 0.f;  // reference max (base 2) of row my_q; this lane's half of its sum
+  const float c = neg ? -a.scale_log2 : a.scale_log2;
+  // last key of row my_q, relative to this lane's column group
+  int lim = a.Skv - 1;
+  if (a.causal) lim = min(lim, my_q + off);
+  lim -= 4 * (lane >> 5);
 
   if (nkv > 0) {
     dma(0);
@@ -326,6 +437,7 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     // 32x32 tiles)
     f32x16 s[2];
     if constexpr (mmode != 0) {
+      mask_pack(j);
       mask_init(s);
     } else {
 #pragma unroll
@@ -352,55 +464,50 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       __builtin_amdgcn_sched_barrier(0);
     }
 
-    // base-2 scores with masking; element 4q + e of tile t is key
-    // kv0 + 32 t + 8 q + 4 (lane >> 5) + e
+    if constexpr (mmode != 0)
+      if (j + 1 < nkv) mask_issue(j + 1);
+    // keys past the end or past the causal limit; element 4q + e of half t is
+    // key kv0 + 32 t + 8 q + 4 (lane >> 5) + e
     const int kv0 = j * BN;
-    const bool full = kv0 + BN <= a.Skv && a.mask_dtype < 0 &&
-                      (a.causal == 0 || kv0 + BN - 1 <= qw + off);
+    if (kv0 + BN > a.Skv || (a.causal && kv0 + BN - 1 > qw + off)) {
+      const int rel = lim - kv0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[t][e] = 32 * t + 8 * (e >> 2) + (e & 3) <= rel ? s[t][e] : neg_inf();
+    }
+
+    // online softmax of row my_q (lanes l and l ^ 32 hold its two halves), its
+    // reference max raised only past 2^8 of it (see k_flash_attn): O is
+    // rescaled, and the halves exchange their maxima, almost never
+    const float th = max32(s) * c;
+    if (__any(th > m_i + 8.f)) {
+      const float tmax = fmaxf(th, __shfl_xor(th, 32, 64));
+      const bool up = tmax > m_i + 8.f;
+      const float alpha = up ? fast_exp2(m_i - tmax) : 1.f;
+      m_i = up ? tmax : m_i;
+      l_i *= alpha;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+    }
+    const float mb = m_i == neg_inf() ? 0.f : m_i;  // fully masked so far: P = 0
     float x[2][16];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) x[t][e] = s[t][e] * a.scale_log2;
-    if constexpr (mmode != 0)
-      if (j + 1 < nkv) mask_issue(j + 1);
-    if (!full) {
+      for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(fmaf(s[t][e], c, -mb));
+    {
+      float r[16];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int e = 0; e < 16; ++e) r[e] = x[0][e] + x[1][e];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int kv = kv0 + 32 * t + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-          bool ok = kv < a.Skv && my_q < a.Sq;
-          if (a.causal) ok = ok && kv <= my_q + off;
-          x[t][e] = ok ? x[t][e] : neg_inf();
-        }
+      for (int w = 8; w >= 1; w >>= 1)
+#pragma unroll
+        for (int e = 0; e < w; ++e) r[e] += r[e + w];
+      l_i += r[0];
     }
-
-    // online softmax of row my_q (lanes l and l ^ 32 hold its two halves)
-    float mx = neg_inf();
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, x[t][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_i, mx);
-    const float m_use = m_new == neg_inf() ? 0.f : m_new;  // fully masked so far: keep P = 0
-    const float alpha = fast_exp2(m_i - m_use);
-    float rs = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        x[t][e] = fast_exp2(x[t][e] - m_use);
-        rs += x[t][e];
-      }
-    rs += __shfl_xor(rs, 32, 64);
-    l_i = l_i * alpha + rs;
-    m_i = m_new;
-#pragma unroll
-    for (int t = 0; t < DT; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
 
     // O += P V over the four 16-key slices, hand-pipelined as S above
     {
@@ -424,7 +531,9 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     // tile j + 1 landed (the next tile's mask loads, issued after it, may
     // still be in flight)
     if (j + 1 < nkv) {
-      if constexpr (mmode == 1)
+      if (kWide && tile_in(j + 1))
+        wait_vmcnt<2 * esz>();
+      else if (mmode == 1 || (mmode == 2 && tile_in(j + 1)))
         wait_vmcnt<8>();
       else if constexpr (mmode == 2)
         wait_vmcnt<32>();
@@ -434,6 +543,7 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     __syncthreads();
   }
 
+  l_i += __shfl_xor(l_i, 32, 64);
   if (my_q >= a.Sq) return;
   const float inv = l_i > 0.f ? 1.f / l_i : 0.f;
   T* O = static_cast<T*>(a.o) + b * a.os[0] + h * a.os[1] + static_cast<int64_t>(my_q) * a.os[2];
@@ -707,22 +817,7 @@ __global__ __launch_bounds__(512, 1) void k_flash_attn(AttnArgs a, int nqb) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[u][e] = 32 * u + 8 * (e >> 2) + (e & 3) <= rel ? s[u][e] : neg_inf();
     }
-    // max of this lane's half of the row: 16 three-way maxima in a tree
-    float mh;
-    {
-      float v[32];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[16 * u + e] = s[u][e];
-      float m1[11];
-#pragma unroll
-      for (int i = 0; i < 10; ++i) m1[i] = max3(v[3 * i], v[3 * i + 1], v[3 * i + 2]);
-      m1[10] = max3(v[30], v[31], v[31]);
-      const float m2a = max3(m1[0], m1[1], m1[2]), m2b = max3(m1[3], m1[4], m1[5]);
-      const float m2c = max3(m1[6], m1[7], m1[8]), m2d = max3(m1[9], m1[10], m1[10]);
-      mh = max3(m2a, m2b, max3(m2c, m2d, m2d));
-    }
+    const float mh = max32(s);
     const float th = mh * c;  // max of this lane's half of the row (base 2)
     if (__any(th > m_run + 8.f)) {
       const float tmax = fmaxf(th, __shfl_xor(th, 32, 64));
@@ -1187,13 +1282,15 @@ int run_attention(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st)
     const bool mask_fits = a.mask_dtype < 0 ||
                            (a.ms[3] == 1 && a.scale_log2 != 0.f &&
                             (static_cast<int64_t>(a.Sq) * a.ms[2] + a.Skv + 68) * esz < 0x7fffffffLL);
-    if (mfma && mask_fits) {
+    if (mfma && mask_fits && (a.scale_log2 > 0.f || a.scale_log2 < 0.f)) {
       const int nqb = (a.Sq + 127) / 128;
       const int64_t total = static_cast<int64_t>(nqb) * a.Hq * a.B;
       if (total > 0x7fffffffLL) return set_error(NTOPS_ERR_UNSUPPORTED, "sdpa: too many blocks");
       const uintptr_t mp = reinterpret_cast<uintptr_t>(a.mask);
       const int mm = a.mask_dtype < 0 ? 0
-                     : (a.ms[2] % 4 == 0 && a.ms[1] % 4 == 0 && a.ms[0] % 4 == 0 && mp % (4 * esz) == 0) ? 1 : 2;
+                     // (a run that straddles the last key would reach past
+                     // the plane in its last row, and read as zero there)
+                     : (a.Skv % 4 == 0 && a.ms[2] % 4 == 0 && a.ms[1] % 4 == 0 && a.ms[0] % 4 == 0 && mp % (4 * esz) == 0) ? 1 : 2;
       const dim3 grid = blocks_2d(total), block(256);
       note_kernel("sdpa_fwd d%d mask%d es%d", a.D > 64 ? 128 : 64, mm, esz);
 #define NTOPS_FWD(DD, MM, ES) hipLaunchKernelGGL((k_flash_fwd<T, DD, MM, ES>), grid, block, 0, st, a, nqb, static_cast<int>(total))

@@ -370,11 +370,18 @@ __global__ __launch_bounds__(256) void k_attn_merge(AttnArgs a, int nsplit, cons
 void decode_split(int64_t heads, int Skv, int D, int& waves, int& nsplit, int& chunk) {
   waves = heads < 2 * cu_count_cached() ? 2 : 1;
   const int step = (D > 64 ? 32 : 64) * waves;
-  const int64_t n = std::max<int64_t>(
-      1, std::min({static_cast<int64_t>(kDecodeMaxSplit), cu_count_cached() / heads, ceil_div(Skv, 4 * step)}));
+  int64_t n = std::min({static_cast<int64_t>(kDecodeMaxSplit), cu_count_cached() / heads, ceil_div(Skv, 4 * step)});
+  if (n <= 2 && Skv <= 8 * step) n = 1;  // two short slices gain what the merge's launch costs
+  n = std::max<int64_t>(n, 1);
   chunk = static_cast<int>(ceil_div(ceil_div(Skv, n), step)) * step;
   nsplit = static_cast<int>(ceil_div(Skv, chunk));
 }
+
+// Few heads over a short cache stay on the 128-row kernel: four waves share
+// the tiles of a head there ((8, 32 / 8, 1, 256, 128): 11.8 us, here 14.6);
+// from a head per CU on every byte counts ((32, 32 / 8, 1, 256, 64): 15.6
+// against 10.9 us, (32, 32, 1, 256, 128): 34.8 against 28.8).
+bool decode_pays(int64_t heads, int64_t Skv) { return Skv > kDecodeMinKeys || heads >= cu_count_cached(); }
 
 template <typename T, int D, int NW>
 int launch_decode(const AttnArgs& a, int nsplit, int chunk, float* part, hipStream_t st) {
@@ -414,7 +421,7 @@ int run_decode(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st) {
 bool attn_decode_serves(const AttnArgs& a) {
   const auto rows16 = [](const int64_t* s) { return s[3] == 1 && s[2] % 8 == 0 && s[1] % 8 == 0 && s[0] % 8 == 0; };
   const int64_t ld = std::max(a.ks[2], a.vs[2]);
-  return a.mask_dtype < 0 && a.Skv > kDecodeMinKeys && static_cast<int64_t>(a.Sq) * (a.Hq / a.Hkv) <= 16 &&
+  return a.mask_dtype < 0 && decode_pays(static_cast<int64_t>(a.B) * a.Hkv, a.Skv) && static_cast<int64_t>(a.Sq) * (a.Hq / a.Hkv) <= 16 &&
          a.D % 8 == 0 && a.D <= 128 && rows16(a.qs) && rows16(a.ks) && rows16(a.vs) && a.os[3] == 1 &&
          a.os[2] % 4 == 0 && a.os[1] % 4 == 0 && a.os[0] % 4 == 0 && aligned16(a.q) && aligned16(a.k) &&
          aligned16(a.v) && (reinterpret_cast<uintptr_t>(a.o) & 7u) == 0 && a.ks[2] >= a.D && a.vs[2] >= a.D &&
@@ -423,7 +430,7 @@ bool attn_decode_serves(const AttnArgs& a) {
 }
 
 int64_t attn_decode_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv, int64_t D) {
-  if (Skv <= kDecodeMinKeys || Sq * (Hq / Hkv) > 16 || D % 8 != 0 || D > 128) return 0;
+  if (!decode_pays(B * Hkv, Skv) || Sq * (Hq / Hkv) > 16 || D % 8 != 0 || D > 128) return 0;
   int waves, nsplit, chunk;
   decode_split(B * Hkv, static_cast<int>(Skv), static_cast<int>(D), waves, nsplit, chunk);
   return nsplit > 1 ? B * Hq * Sq * nsplit * (D + 2) * 4 : 0;

@@ -1,0 +1,69 @@
+"""GPU parity: masked attention on the matrix cores over the mask's load paths
+-- interior tiles by wide loads at any alignment, the partial last tile by runs
+or elements, tiles the mask leaves open -- and the scale's sign."""
+
+import pytest
+import torch
+
+import ntops_amd
+from ntops_amd import _lib
+from oracle import ops as O
+from tests.helpers import DT_NAME, assert_close, from_np, to_np
+
+pytestmark = [
+    pytest.mark.gpu,
+    pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU"),
+]
+
+sdpa = ntops_amd.torch.scaled_dot_product_attention
+
+
+def oracle(q, k, v, mask, scale=None):
+    dt = DT_NAME[q.dtype]
+    m = None if mask is None else to_np(mask.contiguous())
+    return from_np(O.scaled_dot_product_attention(to_np(q), to_np(k), to_np(v), dt, m,
+                                                  None if mask is None else DT_NAME[mask.dtype], 0, scale,
+                                                  round_p=True), dt)
+
+
+# one tile exactly, one key past and short of a tile, several tiles with odd
+# remainders; rows of a wider mask starting at an odd element
+@pytest.mark.parametrize("skv", (1, 63, 64, 65, 130, 191, 256, 333))
+@pytest.mark.parametrize("mask_dtype", (torch.bool, torch.float16, torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("offset", (0, 1, 4))
+def test_mask_loads(skv, mask_dtype, offset):
+    g = torch.Generator().manual_seed(skv + offset)
+    dtype, b, h, sq, d = torch.float16 if skv % 2 else torch.bfloat16, 2, 3, 70, 64
+    q, k, v = (torch.randn(b, h, s, d, generator=g).to(dtype) for s in (sq, skv, skv))
+    keep = torch.rand(b, 1, sq, skv + offset + 3, generator=g) > 0.3
+    keep[:, :, :40, :128] = True   # open tiles beside mixed ones
+    keep[0, :, 5] = False          # a row with no key
+    keep[1, :, 7, 64:] = False
+    mask = keep if mask_dtype == torch.bool else torch.where(keep, 0.25 * torch.rand(keep.shape, generator=g).round(),
+                                                             float("-inf")).to(mask_dtype)
+    mask = mask[..., offset:offset + skv]
+    wide = torch.zeros(b, 1, sq, skv + offset + 3).to(mask_dtype).cuda()
+    wide[..., offset:offset + skv] = mask.cuda()
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=wide[..., offset:offset + skv])
+    assert _lib.last_kernel().startswith("sdpa_fwd d64 mask"), _lib.last_kernel()
+    full = mask.expand(b, h, sq, skv)
+    assert_close(got, oracle(q, k, v, full), 1.6e-2, 1.6e-2, "mask")
+    assert (got[0, :, 5] == 0).all()
+    # the same under a padding mask that no query row moves
+    pad = mask[:, :, 9:10]
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=wide[:, :, 9:10, offset:offset + skv])
+    assert_close(got, oracle(q, k, v, pad.expand(b, h, sq, skv)), 1.6e-2, 1.6e-2, "padding")
+
+
+@pytest.mark.parametrize("scale", (-0.2, 0.0, 3.0))
+@pytest.mark.parametrize("masked", (False, True))
+def test_scale_signs(scale, masked):
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(1, 2, s, 128, generator=g).bfloat16() for s in (20, 150, 150))
+    mask = None
+    if masked:
+        mask = torch.where(torch.rand(20, 150, generator=g) > 0.5, 0.0, -1.5)
+        mask[:, 30:40] = float("-inf")
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=None if mask is None else mask.cuda(), scale=scale)
+    exp = oracle(q, k, v, None if mask is None else mask.expand(1, 2, 20, 150), scale)
+    assert_close(got, exp, 1.6e-2, 1.6e-2, f"scale {scale}")
