@@ -588,10 +588,29 @@ int skinny_j(int64_t M, int64_t N, int64_t batch) {
   return 1;
 }
 
+// Whether a K-major B of a product of up to 16 rows is streamed by the DMA
+// kernel: from 96 MiB, a size that the 256 MB Infinity Cache does not keep
+// between two uses by a program with other data.  Measured at 8 rows, register
+// kernel -> DMA kernel, B from memory: 14336 x 4096 bf16 (117 MB) 28.8 -> 22.7
+// us, 4096 x 14336 32.5 -> 22.1, 8192 x 28672 109.6 -> 76.1, 32000 x 4096 56.4
+// -> 47.3, 10240 x 8192 50.9 -> 43.1; fp32 14336 x 4096 53.2 -> 46.7, 4096 x
+// 14336 60.4 -> 39.7, 50257 x 768 41.4 -> 35.9.  Below the line the two are
+// level on a B from memory (11008 x 4096 bf16, 90 MB: 27.6 -> 26.3; 50257 x
+// 768 22.0 -> 22.2), and the register kernel, with several blocks per CU, is
+// faster on one that the cache still holds (23.2 -> 25.9; 17.5 -> 21.7).
+bool skinny_streams(const GemmArgs& g, int es) {
+  const int64_t copies = g.sb_b == 0 ? 1 : g.batch;
+  return static_cast<int64_t>(g.N) * g.K * es * copies >= (int64_t(96) << 20);
+}
+
 template <typename T, bool BKM>
 int launch_skinny(const GemmArgs& g, hipStream_t st) {
   const int mb = (g.M + 15) / 16;
   const int j = skinny_j(g.M, g.N, g.batch);
+  if (BKM && mb == 1 && skinny_streams(g, sizeof(T))) {
+    note_kernel("gemm_skinny m16 n%d B:K dma", 16 * j);
+    return gemm_skinny_dma(std::is_same<T, __bf16>::value ? NTOPS_BF16 : NTOPS_F16, g, j, st);
+  }
   if (mb == 1) return launch_skinny_mb<T, BKM, 1>(g, st, j);
   if (mb == 2) return launch_skinny_mb<T, BKM, 2>(g, st, j);
   if (mb == 3) return launch_skinny_mb<T, BKM, 3>(g, st, j);
@@ -749,6 +768,10 @@ int launch_skinny_f32(const GemmArgs& g, hipStream_t st) {
       j = c;
       break;
     }
+  }
+  if (BKM && mb == 1 && skinny_streams(g, 4)) {
+    note_kernel("gemm_skinny_f32 m16 n%d B:K dma", 16 * j);
+    return gemm_skinny_dma(NTOPS_F32, g, j, st);
   }
   if (mb == 1) return launch_skinny_f32_mb<BKM, 1>(g, st, j);
   if (mb == 2) return launch_skinny_f32_mb<BKM, 2>(g, st, j);

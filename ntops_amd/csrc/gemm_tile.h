@@ -532,6 +532,10 @@ __device__ __forceinline__ void store_tile_direct(const GemmArgs& g, const f32x1
 constexpr bool kStreamOutMfma = true;
 constexpr bool kStreamOutPanel = true;
 
+// Up to 16 rows with a K-major A and B in 16-byte rows, 16 j columns per block
+// (gemm_skinny.hip).
+int gemm_skinny_dma(int dtype, const GemmArgs& g, int j, hipStream_t st);
+
 // The 256 x 256 persistent kernel (gemm_large.hip): 16-bit products in the
 // matrix-core layouts (see run_gemm) that gemm_large_serves.
 bool gemm_large_serves(const GemmArgs& g);
