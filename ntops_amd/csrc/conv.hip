@@ -88,6 +88,7 @@ struct ConvArgs {
   int64_t xs[4], ws[4], os[4], bs;
   int N, C, H, W, K, R, S, P, Q;
   int sh, sw, ph, pw, dh, dw;
+  int block;  // channels-last GEMM: channels per K tile (32 or 64)
 };
 
 // Output plane rows of pq pixels from rows of ld pixels (image i, channel
@@ -456,22 +457,23 @@ __global__ __launch_bounds__(256) void k_conv_to_cl(ConvArgs a, T* xt, int n0, i
   }
 }
 
-// Weights in the channels-last GEMM's k order (32-channel blocks, then
-// taps, then the block's channels): wt[k][((cb * R + r) * S + s) * 32 + ci]
-// = w[k][32 cb + ci][r][s].  Item i (of K C R S / 8) is 8 channels: 8
+// Weights in the channels-last GEMM's k order (blocks of a.block channels,
+// 32 here, then taps, then the block's channels): wt[k][((cb * R + r) * S + s)
+// * 32 + ci] = w[k][32 cb + ci][r][s].  Item i (of K C R S / 8) is 8 channels: 8
 // loads, one 16-byte store.
 template <typename T>
 __device__ __forceinline__ void conv_weight_pack(const ConvArgs& a, T* wt, int64_t i) {
   const T* w = static_cast<const T*>(a.w);
-  const int ci8 = static_cast<int>(i % 4) * 8;  // the 8 channels' offset in the block
-  int64_t t = i / 4;
+  const int items = a.block / 8;
+  const int ci8 = static_cast<int>(i % items) * 8;  // the 8 channels' offset in the block
+  int64_t t = i / items;
   const int s = static_cast<int>(t % a.S);
   t /= a.S;
   const int r = static_cast<int>(t % a.R);
   t /= a.R;
-  const int cb = static_cast<int>(t % (a.C / 32));
-  const int k = static_cast<int>(t / (a.C / 32));
-  const T* src = w + k * a.ws[0] + static_cast<int64_t>(cb * 32 + ci8) * a.ws[1] + r * a.ws[2] + s * a.ws[3];
+  const int cb = static_cast<int>(t % (a.C / a.block));
+  const int k = static_cast<int>(t / (a.C / a.block));
+  const T* src = w + k * a.ws[0] + static_cast<int64_t>(cb * a.block + ci8) * a.ws[1] + r * a.ws[2] + s * a.ws[3];
   T v[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = src[e * a.ws[1]];
@@ -828,6 +830,8 @@ extern "C" int ntops_conv2d(int dtype, int64_t N, int64_t C, int64_t H, int64_t 
     const int64_t nb_max = std::min<int64_t>(N, (workspace_bytes - fixed) / per_image);
     void* wt = workspace;
     void* xt = static_cast<char*>(workspace) + fixed;
+    // one order of the weights for all chunks, by the full ones' size
+    a.block = conv_large_serves(nb_max, K, P * Q, C, R, S, Q, out_strides[1], bias, bias_stride) ? 64 : 32;
     // 16-byte input rows: the block copy, which also reorders the weights
     // (with the first chunk); otherwise the element copy after a weight launch
     const bool rows16 = a.xs[3] == 1 && a.xs[2] % 8 == 0 && a.xs[1] % 8 == 0 && a.xs[0] % 8 == 0 &&
@@ -869,7 +873,8 @@ extern "C" int ntops_conv2d(int dtype, int64_t N, int64_t C, int64_t H, int64_t 
                                    static_cast<int>(crs), wt, xt, img, static_cast<int>(R), static_cast<int>(S),
                                    static_cast<int>(C), static_cast<int>(Q), static_cast<int>(stride_h),
                                    static_cast<int>(stride_w), static_cast<int>(wp), static_cast<int>(dil_h),
-                                   static_cast<int>(dil_w), bias, bias_stride, dst, out_strides[0], out_strides[1], st);
+                                   static_cast<int>(dil_w), bias, bias_stride, dst, out_strides[0], out_strides[1], a.block,
+                                   st);
       if (rc != NTOPS_OK) return rc;
     }
     return NTOPS_OK;

@@ -1575,7 +1575,7 @@ int gemm_implicit_conv(int dtype, int batch, int M, int N, int K, const void* w,
 int gemm_conv_channels_last(int dtype, int batch, int M, int N, int K, const void* w, const void* xt,
                             int64_t img_elems, int R, int S, int C, int Q, int sh, int sw, int wp, int dh,
                             int dw, const void* bias, int64_t bias_stride, void* out, int64_t out_batch,
-                            int64_t out_ld, hipStream_t st) {
+                            int64_t out_ld, int block, hipStream_t st) {
   if (batch <= 0 || M <= 0 || N <= 0 || K <= 0) return NTOPS_OK;
   if (!aligned16(w) || !aligned16(xt) || C % 32 || K != R * S * C || N % 4 || img_elems % 8 || out_ld % 4 ||
       out_batch % 4 || (reinterpret_cast<uintptr_t>(out) & 7u))
@@ -1620,6 +1620,7 @@ int gemm_conv_channels_last(int dtype, int batch, int M, int N, int K, const voi
   g.cl_c = C;
   g.cl_dh = dh;
   g.cl_dw = dw;
+  if (block == 64) return gemm_conv_large(dtype, g, st);
   switch (dtype) {
     case NTOPS_BF16: return run_implicit_conv<__bf16, 2>(g, st);
     case NTOPS_F16: return run_implicit_conv<_Float16, 2>(g, st);

@@ -29,8 +29,17 @@
 // Same-box pairs, before (32-deep K tiles, one block per tile) and now, bf16:
 // 8192 x 14336 x 4096 766 -> 640 us (K-major B; the matrix library 622), 717
 // -> 655 (N-major B; 720); 4096^3 108 -> 93; 6000 x 6000 x 4096 388 -> 245.
+//
+// The channels-last convolution (PixelLoader) runs on the same kernel: a K
+// tile is a 64-channel block under one tap, so a pixel's piece is one whole
+// 128-byte line (the 32-channel kernel fetched halves of them), and a tile's
+// stores leave under the next one's MFMAs.  Whole conv2d calls, bf16 3 x 3:
+// (32, 256, 56, 56) to 256 148.7 -> 122.1 us, (32, 128, 56, 56) to 128 75.2 ->
+// 64.8, (32, 64, 112, 112) to 128 152.8 -> 136.2.  What is left there is the
+// input's copy (19 us) and 416 tiles over 256 CUs: two rounds, 0.8 full.
 #include <algorithm>
 
+#include "gemm.h"
 #include "gemm_tile.h"
 
 namespace ntops {
@@ -153,6 +162,45 @@ struct HalfLoader {
   }
 };
 
+// The same for a channels-last convolution's pixels (see GemmArgs): a K tile
+// is one 64-channel block under one tap, a row one output pixel.
+struct PixelLoader {
+  uint32_t lds_off;
+
+  // this lane's chunk of its row for instruction i, in elements
+  __device__ __forceinline__ static int lane_k(int wave, int lane, int i) {
+    return HalfLoader<true>::lane_k(wave, lane, i);
+  }
+  __device__ __forceinline__ void init(int64_t, int wave, int) { lds_off = static_cast<uint32_t>(wave * 2048); }
+  // Byte offset of this lane's chunk of pixel nh + row under the first tap of
+  // the first block (pixels past the image read its last one's: columns that
+  // are never stored).  n / cl_q by multiplication, exact on the sizes that
+  // conv_large_serves takes.
+  __device__ __forceinline__ static uint32_t pixel(const GemmArgs& g, int nh, int wave, int lane, int i) {
+    const uint32_t n = static_cast<uint32_t>(min(nh + (wave * 2 + i) * 8 + lane / 8, g.N - 1));
+    const uint32_t p = __umulhi(n, g.cl_mq);
+    const uint32_t col = static_cast<uint32_t>(g.cl_sw) * g.cl_c;
+    const uint32_t row = static_cast<uint32_t>(g.cl_sh) * g.cl_wp * g.cl_c;
+    return (n * col + p * (row - g.cl_q * col) + lane_k(wave, lane, i)) * 2;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ void issue(u32x4 rsrc, uint32_t lds, const uint32_t (&pix)[2], int t, const GemmArgs& g) const {
+    const uint32_t ut = static_cast<uint32_t>(t);
+    const uint32_t cb = (ut * g.cl_mrs) >> 16;  // channel block and tap of the K tile
+    const uint32_t tap = ut - cb * g.cv_rs;
+    const uint32_t r = (tap * g.cl_ms) >> 16;
+    const uint32_t c = tap - r * g.cv_s;
+    uint32_t koff = ((r * g.cl_dh * g.cl_wp + c * g.cl_dw) * g.cl_c + cb * 64) * 2;
+    asm volatile("" : "+s"(koff));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t off = pix[i] + koff;
+      if constexpr (TAIL) off = t * 64 < g.K ? off : kOOB;
+      dma16(rsrc, lds + lds_off + i * 1024, off);
+    }
+  }
+};
+
 __device__ __forceinline__ u32x4 make_rsrc(const void* base, int64_t bytes) {
   const uint64_t addr = reinterpret_cast<uint64_t>(base);
   u32x4 r;
@@ -165,9 +213,11 @@ __device__ __forceinline__ u32x4 make_rsrc(const void* base, int64_t bytes) {
 
 // Resources of an output tile's operand halves (what lies past an edge reads
 // as zero, or as some other row's or column's data: such rows and columns of
-// the product are never stored).
+// the product are never stored); a convolution's pixel offsets.
+template <bool CONV>
 struct TileRsrc {
   u32x4 a[2], b[2];
+  uint32_t pix[CONV ? 2 : 1][2];  // [column half][instruction]
 };
 
 template <int N>
@@ -175,8 +225,11 @@ __device__ __forceinline__ void wait_vm() {
   wait_vmcnt<(N < 63 ? N : 63)>();
 }
 
-template <typename T, bool AK, bool BKM, bool BIAS>
+// CONV: B is the channels-last convolution operand, the bias a value per row.
+template <typename T, bool AK, bool BKM, bool BIAS, bool CONV = false>
 __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
+  static_assert(!CONV || (AK && BKM), "the convolution's operands are K-major");
+  using Rsrc = TileRsrc<CONV>;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -206,7 +259,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
     return true;
   };
   auto rsrc_of = [&](bool ok, int bat, int m0, int n0) __attribute__((always_inline)) {
-    TileRsrc r;
+    Rsrc r;
     const uint16_t* A = static_cast<const uint16_t*>(g.A) + bat * g.sa_b;
     const uint16_t* B = static_cast<const uint16_t*>(g.B) + bat * g.sb_b;
 #pragma unroll
@@ -216,6 +269,12 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
       r.a[h] = mv <= 0 ? make_rsrc(g.A, 0)
                : AK    ? make_rsrc(A + static_cast<int64_t>(mh) * g.sa_m, (static_cast<int64_t>(mv - 1) * g.sa_m + g.K) * 2)
                        : make_rsrc(A + mh, (static_cast<int64_t>(g.K - 1) * g.sa_k + mv) * 2);
+      if constexpr (CONV) {  // the batch's whole padded image
+        r.b[h] = make_rsrc(B, nv > 0 ? g.sb_b * 2 : 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) r.pix[h][i] = PixelLoader::pixel(g, nh, wave, here(lane), i);
+        continue;
+      }
       r.b[h] = nv <= 0 ? make_rsrc(g.B, 0)
                : BKM   ? make_rsrc(B + static_cast<int64_t>(nh) * g.sb_n, (static_cast<int64_t>(nv - 1) * g.sb_n + g.K) * 2)
                        : make_rsrc(B + nh, (static_cast<int64_t>(g.K - 1) * g.sb_k + nv) * 2);
@@ -224,23 +283,26 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
   };
 
   HalfLoader<AK> la;
-  HalfLoader<BKM> lb;
+  std::conditional_t<CONV, PixelLoader, HalfLoader<BKM>> lb;
   la.init(AK ? g.sa_m : g.sa_k, wave, lane);
   lb.init(BKM ? g.sb_n : g.sb_k, wave, lane);
   const uint32_t smem_addr = lds_addr(smem);
 
   int bat, m0, n0, nbat = 0, nm0 = 0, nn0 = 0;
   if (!tile_at(0, bat, m0, n0)) return;  // (the whole block)
-  TileRsrc cur = rsrc_of(true, bat, m0, n0), nxt;
+  Rsrc cur = rsrc_of(true, bat, m0, n0), nxt;
 
   // loads of half tile `half` of operand A / B of K tile t (buffer t & 1)
-  auto dma_a = [&](auto tail, const TileRsrc& rs, int half, int t) __attribute__((always_inline)) {
+  auto dma_a = [&](auto tail, const Rsrc& rs, int half, int t) __attribute__((always_inline)) {
     la.template issue<decltype(tail)::value>(
         rs.a[half], smem_addr + static_cast<uint32_t>(((t & 1) * 2 + half) * kHalf), t * 64, g.K, wave, lane);
   };
-  auto dma_b = [&](auto tail, const TileRsrc& rs, int half, int t) __attribute__((always_inline)) {
-    lb.template issue<decltype(tail)::value>(
-        rs.b[half], smem_addr + static_cast<uint32_t>(kAreaB + ((t & 1) * 2 + half) * kHalf), t * 64, g.K, wave, lane);
+  auto dma_b = [&](auto tail, const Rsrc& rs, int half, int t) __attribute__((always_inline)) {
+    const uint32_t lds = smem_addr + static_cast<uint32_t>(kAreaB + ((t & 1) * 2 + half) * kHalf);
+    if constexpr (CONV)
+      lb.template issue<decltype(tail)::value>(rs.b[half], lds, rs.pix[half], t, g);
+    else
+      lb.template issue<decltype(tail)::value>(rs.b[half], lds, t * 64, g.K, wave, lane);
   };
 
   f32x4 acc[4][2][4];  // [quadrant][row tile][column tile]
@@ -272,12 +334,13 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
   bool pend = false;
   auto row_half = [&](int q) __attribute__((always_inline)) { return q == 1 || q == 2; };
   auto col_half = [&](int q) __attribute__((always_inline)) { return q >= 2; };
-  // the bias columns of the tile at n: lanes 0-31 the first half's, 32-63 the
+  // the bias columns of the tile at n (CONV: rows at m): lanes 0-31 the first half's, 32-63 the
   // second's, two per lane (past N: zero; an odd N's last pair is one dword)
-  auto bias_dma = [&](int n) __attribute__((always_inline)) {
+  auto bias_dma = [&](int m, int n) __attribute__((always_inline)) {
     const int l = here(lane);
-    const uint32_t off = static_cast<uint32_t>((n + (l >> 5) * 128 + wn * 64 + (l & 31) * 2) * 2);
-    const u32x4 r = make_rsrc(g.C, (static_cast<int64_t>(g.N) * 2 + 3) & ~3ll);
+    const uint32_t off = CONV ? static_cast<uint32_t>((m + (l >> 5) * 128 + wm * 32 + (l & 15) * 2) * 2)
+                              : static_cast<uint32_t>((n + (l >> 5) * 128 + wn * 64 + (l & 31) * 2) * 2);
+    const u32x4 r = make_rsrc(g.C, (static_cast<int64_t>(CONV ? g.M : g.N) * 2 + 3) & ~3ll);
     asm volatile("buffer_load_dword %0, %1, 0 offen lds" : : "v"(off), "s"(r), "{m0}"(bias_lds) : "memory");
   };
   // LDS address of this lane's 4 columns in column tile 0; column tile ct
@@ -286,10 +349,20 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
     const int r = l & 15, c = l >> 5, half = (l >> 4) & 1;
     return ep + static_cast<uint32_t>(r * 128 + ((c ^ (r >> 1)) << 4) + half * 8);
   };
-  // the bias values of column tile ct of quadrant q for this lane
+  // the bias values of quadrant q for this lane: per column tile its 4
+  // columns', CONV: per row tile its row's
   typedef __attribute__((address_space(3))) const u32x2 lds_cu32x2_t;
-  auto bias_of = [&](int q, int ct, int l) __attribute__((always_inline)) {
-    return *reinterpret_cast<lds_cu32x2_t*>(bias_lds + static_cast<uint32_t>(col_half(q) * 128 + ct * 32 + (l >> 4) * 8));
+  typedef __attribute__((address_space(3))) const uint16_t lds_cu16_t;
+  auto bias_of = [&](int q, int l, u32x2 (&bias)[4]) __attribute__((always_inline)) {
+    if constexpr (CONV) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+        bias[rt].x = *reinterpret_cast<lds_cu16_t*>(bias_lds + static_cast<uint32_t>(row_half(q) * 128 + rt * 32 + (l & 15) * 2));
+    } else {
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct)
+        bias[ct] = *reinterpret_cast<lds_cu32x2_t*>(bias_lds + static_cast<uint32_t>(col_half(q) * 128 + ct * 32 + (l >> 4) * 8));
+    }
   };
   // rounds row tile i / 4, column tile i % 4 of quadrant q into the staging
   auto convert = [&](int q, int i, uint32_t base, const u32x2 (&bias)[4]) __attribute__((always_inline)) {
@@ -298,10 +371,10 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = acc[q][rt][ct][e];
     if constexpr (BIAS) {
-      const u32x2 raw = bias[ct];
+      const u32x2 raw = bias[CONV ? rt : ct];
       const T* t = reinterpret_cast<const T*>(&raw);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = g.alpha * v[e] + g.beta * static_cast<float>(t[e]);
+      for (int e = 0; e < 4; ++e) v[e] = g.alpha * v[e] + g.beta * static_cast<float>(t[CONV ? 0 : e]);
     }
     T o[4];
 #pragma unroll
@@ -364,23 +437,20 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
     }
   };
 
-  // the quadrant's 16 MFMAs; CONV: finished quadrant cq leaves between them --
+  // the quadrant's 16 MFMAs; LEAVE: finished quadrant cq leaves between them --
   // its first row tile's rows are stored under its second's conversion, its
   // second's are left in `rows` (put_rows by the caller)
   u32x4 rows[2];
-  auto mfma16x = [&](auto first, auto conv, int q, const u32x4 (&af)[4], int cq) __attribute__((always_inline)) {
-    constexpr bool FIRST = decltype(first)::value, CONV = decltype(conv)::value;
+  auto mfma16x = [&](auto first, auto leave, int q, const u32x4 (&af)[4], int cq) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first)::value, LEAVE = decltype(leave)::value;
     int l = 0;
     uint32_t base = 0;
     u32x2 bias[4];
-    if constexpr (CONV) {
+    if constexpr (LEAVE) {
       l = here(lane);
       base = ep_base(l);
       scale(cq);
-      if constexpr (BIAS) {
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) bias[ct] = bias_of(cq, ct, l);
-      }
+      if constexpr (BIAS) bias_of(cq, l, bias);
     }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
@@ -391,7 +461,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
           f32x4 c = acc[q][rt][ct];
           if (FIRST && ks == 0) c = f32x4{0.f, 0.f, 0.f, 0.f};
           acc[q][rt][ct] = mfma16<T>(bx[ct][ks], af[ks * 2 + rt], c);
-          if constexpr (CONV) {
+          if constexpr (LEAVE) {
             const int i = ks * 8 + rt * 4 + ct;  // piece i / 2 after every second MFMA
             if (i & 1) {
               __builtin_amdgcn_sched_barrier(0);
@@ -432,7 +502,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
   // The waits allow for the 8 loads issued since the ones the next phase
   // reads, plus the stores among them while a tile leaves (two per put_rows:
   // 4, 8, 5 and 1 of them).
-  auto ktile = [&](auto kind_tag, auto buf_tag, auto tail, const TileRsrc& rs1, int t1, const TileRsrc& rs2,
+  auto ktile = [&](auto kind_tag, auto buf_tag, auto tail, const Rsrc& rs1, int t1, const Rsrc& rs2,
                    int t2) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind_tag)::value, BUF = decltype(buf_tag)::value;
     constexpr auto first = std::bool_constant<KIND == 0>{};
@@ -500,7 +570,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
     // the loads of the last two K tiles, which may reach past K
     ktile(NTOPS_W(1), b0, yes, cur, t + 1, cur, t + 2);
     ktile(NTOPS_W(1), b1, yes, cur, t + 2, cur, t + 3);
-    if constexpr (BIAS) bias_dma(n0);
+    if constexpr (BIAS) bias_dma(m0, n0);
     const bool more = tile_at(it + 1, nbat, nm0, nn0);
     nxt = rsrc_of(more, nbat, nm0, nn0);
     ktile(NTOPS_W(1), b0, yes, cur, t + 3, nxt, 0);
@@ -518,10 +588,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
   for (int q = 2; q < 4; ++q) {
     scale(q);
     u32x2 bias[4];
-    if constexpr (BIAS) {
-#pragma unroll
-      for (int ct = 0; ct < 4; ++ct) bias[ct] = bias_of(q, ct, lane);
-    }
+    if constexpr (BIAS) bias_of(q, lane, bias);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
 #pragma unroll
@@ -533,9 +600,9 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
   wait_vmcnt<0>();  // no DMA may land after the workgroup ends
 }
 
-template <typename T, bool AK, bool BKM, bool BIAS>
+template <typename T, bool AK, bool BKM, bool BIAS, bool CONV = false>
 int launch_large(const GemmArgs& g, hipStream_t st) {
-  auto kern = k_gemm_large<T, AK, BKM, BIAS>;
+  auto kern = k_gemm_large<T, AK, BKM, BIAS, CONV>;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -561,6 +628,11 @@ int run_large(bool ak, bool bk, const GemmArgs& g, hipStream_t st) {
   return bk ? launch_large_c<T, false, true>(g, st) : launch_large_c<T, false, false>(g, st);
 }
 
+template <typename T>
+int run_conv_large(const GemmArgs& g, hipStream_t st) {
+  return g.use_c ? launch_large<T, true, true, true, true>(g, st) : launch_large<T, true, true, false, true>(g, st);
+}
+
 }  // namespace
 
 bool gemm_large_serves(const GemmArgs& g) {
@@ -576,6 +648,31 @@ bool gemm_large_serves(const GemmArgs& g) {
 int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipStream_t st) {
   return dtype == NTOPS_BF16 ? run_large<__bf16>(a_kmajor, b_kmajor, g, st)
                              : run_large<_Float16>(a_kmajor, b_kmajor, g, st);
+}
+
+// Where the plain kernel's rule holds (240 tiles, K > 256), on images whose
+// channels are whole 64-deep K tiles, with no bias or a contiguous one.  The
+// index divisions by multiplication need
+//  * n / Q: ceil(2^32 / Q) is less than Q too large per 2^32, so the quotient
+//    is exact where n Q < 2^32 (Q = 1: the factor would not fit);
+//  * t / (R S) of K tile t (up to 4 past the last) and tap / S likewise, over
+//    2^16.
+bool conv_large_serves(int64_t images, int64_t M, int64_t pixels, int64_t C, int64_t R, int64_t S, int64_t Q,
+                       int64_t out_ld, const void* bias, int64_t bias_stride) {
+  const int64_t rs = R * S;
+  const bool bias_ok = bias == nullptr || (bias_stride == 1 && M % 2 == 0 && (reinterpret_cast<uintptr_t>(bias) & 3u) == 0);
+  return C % 64 == 0 && C * rs > 256 && bias_ok && Q >= 2 && pixels * Q < (int64_t(1) << 32) &&
+         (C / 64 * rs + 4) * rs < 65536 && rs * S < 65536 && out_ld >= 0 && (16 * out_ld + 64) * 2 < (int64_t(1) << 31) &&
+         ((M + 255) / 256) * ((pixels + 255) / 256) * images >= 240;
+}
+
+int gemm_conv_large(int dtype, GemmArgs g, hipStream_t st) {
+  g.cv_rs = g.cv_r * g.cv_s;
+  g.cl_mq = static_cast<uint32_t>(((uint64_t(1) << 32) + g.cl_q - 1) / g.cl_q);
+  g.cl_mrs = (65536u + g.cv_rs - 1) / g.cv_rs;
+  g.cl_ms = (65536u + g.cv_s - 1) / g.cv_s;
+  note_kernel("gemm_mfma 256x256 s4 A:K B:K %s conv_cl", g.M % 256 == 0 && g.N % 256 == 0 ? "even" : "ragged");
+  return dtype == NTOPS_BF16 ? run_conv_large<__bf16>(g, st) : run_conv_large<_Float16>(g, st);
 }
 
 }  // namespace ntops

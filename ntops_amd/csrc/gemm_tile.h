@@ -45,7 +45,11 @@ struct GemmArgs {
   // s * cl_dw) * cl_c + 32 * cb + ci, so one K tile is one (block, tap) and
   // the R * S tiles of a block, which read overlapping pixels, follow each
   // other (the reuse stays within L2).
+  // The 64-deep kernel (gemm_large.hip) runs over 64-channel blocks instead
+  // and divides by multiplication: ceil(2^32 / cl_q), and ceil(2^16 / d) for
+  // d = cv_rs and cv_s.
   int cl_q, cl_sh, cl_sw, cl_wp, cl_c, cl_dh, cl_dw;
+  uint32_t cl_mq, cl_mrs, cl_ms;
 };
 
 
@@ -540,5 +544,8 @@ int gemm_skinny_dma(int dtype, const GemmArgs& g, int j, hipStream_t st);
 // matrix-core layouts (see run_gemm) that gemm_large_serves.
 bool gemm_large_serves(const GemmArgs& g);
 int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipStream_t st);
+// Its channels-last convolution: k in 64-channel blocks; problems that
+// conv_large_serves (whatever the number of images in one launch).
+int gemm_conv_large(int dtype, GemmArgs g, hipStream_t st);
 
 }  // namespace ntops
