@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
   // past the plane reads 0; such keys are masked anyway).  Tiles that the mask
   // leaves open start from zero.  What this kernel's masked time was before
   // the wide loads, the open tiles and the fused softmax (one fma per score,
-  // three-way maxima, O rescaled only past 2^8), (8, 16, 1000, 64) f16 bool:
+  // three-way maxima, O rescaled only where a max rises), (8, 16, 1000, 64) f16 bool:
   // 118 us -> 79 with the softmax and open tiles -> 62 with the wide loads
   // (float 102 -> 63; (4, 32, 2048, 128) bf16 bool 607 -> 324; rows of 1397
   // keys, read element by element before, 159 -> 71).
@@ -477,13 +477,15 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
         for (int e = 0; e < 16; ++e) s[t][e] = 32 * t + 8 * (e >> 2) + (e & 3) <= rel ? s[t][e] : neg_inf();
     }
 
-    // online softmax of row my_q (lanes l and l ^ 32 hold its two halves), its
-    // reference max raised only past 2^8 of it (see k_flash_attn): O is
-    // rescaled, and the halves exchange their maxima, almost never
+    // online softmax of row my_q (lanes l and l ^ 32 hold its two halves); O is
+    // rescaled, and the halves exchange their maxima, only on tiles that raise
+    // some row's max.  (The max itself stays the reference: a row's largest P
+    // is then 1 and carries no rounding, where a reference raised only past
+    // 2^8 of it, as in k_flash_attn, is 2.5 % further from 64 bits.)
     const float th = max32(s) * c;
-    if (__any(th > m_i + 8.f)) {
+    if (__any(th > m_i)) {
       const float tmax = fmaxf(th, __shfl_xor(th, 32, 64));
-      const bool up = tmax > m_i + 8.f;
+      const bool up = tmax > m_i;
       const float alpha = up ? fast_exp2(m_i - tmax) : 1.f;
       m_i = up ? tmax : m_i;
       l_i *= alpha;
