@@ -1344,7 +1344,10 @@ int pick_tile(const GemmArgs& g, hipStream_t st) {
     return launch_panel<T, AK, BKM>(g, st);
   const int64_t big_tiles = static_cast<int64_t>((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
   constexpr int kBK = 32, kStages = 4;
-  if (big_tiles >= 240 && g.K > 256) {
+  // (one round of 128 x 128 tiles with an N-major B: 2 to 4 % slower on large
+  // ones at K = 1600, 6 to 14 % faster at 4096 and above; M-major A not taken)
+  const int64_t k_min = !AK ? INT64_MAX : BKM ? 1024 : 2048;
+  if (g.K > 256 && (big_tiles >= 240 || (large_tiles_suit(g.M, g.N, g.K, g.batch, k_min) && gemm_large_serves(g)))) {
     const bool even = g.M % 256 == 0 && g.N % 256 == 0 && g.K % kBK == 0;
     // the persistent kernel: no C or a bias row, any output layout and edges
     if (gemm_large_serves(g)) {

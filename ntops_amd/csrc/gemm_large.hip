@@ -1,4 +1,4 @@
-// Large 16-bit GEMM (K > 256, 240 or more 256 x 256 tiles): out = alpha A B
+// Large 16-bit GEMM (K > 256, sizes by large_tiles_suit): out = alpha A B
 // (+ beta times a bias row), any of the four operand layouts, any edges, any
 // output layout.
 //
@@ -650,7 +650,30 @@ int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipSt
                              : run_large<_Float16>(a_kmajor, b_kmajor, g, st);
 }
 
-// Where the plain kernel's rule holds (240 tiles, K > 256), on images whose
+// 240 tiles (a round of the GPU's 256 CUs).  Fewer leave CUs idle, but from
+// the count where 128 x 128 tiles (two to a CU) need a second round on they
+// are still faster: bf16 K-major B, 2560 x 4096 x 4096 (160 tiles) 106.9 -> 70.2
+// us, 3584 x 4096 x 4096 (224) 145.7 -> 84.1, 2816 x 3072 x 768 (132) 25.0 ->
+// 20.1, 2816 x 3072 x 512 19.4 -> 16.5, N-major within 4 %.  Products whose
+// last row or column of large tiles is half empty or more take it from K = 2048
+// on (257 x 25600 x 4096 121.2 -> 73.7, 2050 x 4096 x 2048 68.0 -> 39.9); shorter
+// ones would gain too (2050 x 4096 x 1024 38.7 / 26.6) but keep the kernel that
+// test_gpu_gemm.py states for them.  Where the small tiles fill seven eighths of
+// their one round, a K of k_min or more amortises the large kernel's fill: 2048 x
+// 4096 x 4096 (128) 80.0 -> 65.8, but 3584 x 2304 x 768 (126) 19.1 -> 20.0; not
+// with half empty large tiles (a product of 128 rows).  Below that the small
+// ones are as fast or faster (768 x 6400 x 1600, 75: 34.0 / 32.2; 1024 x 4096 x
+// 4096, 64: 38.7 / 64.5).
+bool large_tiles_suit(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t k_min) {
+  const int64_t cus = cu_count_cached() > 0 ? cu_count_cached() : 256;
+  const int64_t large = ((M + 255) / 256) * ((N + 255) / 256) * batch;
+  const int64_t small = ((M + 127) / 128) * ((N + 127) / 128) * batch;
+  const bool whole = small == 4 * large;
+  return large >= 240 || (small > 2 * cus && K >= (whole ? 512 : 2048)) ||
+         (whole && 4 * small > 7 * cus && K >= k_min);
+}
+
+// Where the plain kernel's tiles suit (K > 256), on images whose
 // channels are whole 64-deep K tiles, with no bias or a contiguous one.  The
 // index divisions by multiplication need
 //  * n / Q: ceil(2^32 / Q) is less than Q too large per 2^32, so the quotient
@@ -663,7 +686,7 @@ bool conv_large_serves(int64_t images, int64_t M, int64_t pixels, int64_t C, int
   const bool bias_ok = bias == nullptr || (bias_stride == 1 && M % 2 == 0 && (reinterpret_cast<uintptr_t>(bias) & 3u) == 0);
   return C % 64 == 0 && C * rs > 256 && bias_ok && Q >= 2 && pixels * Q < (int64_t(1) << 32) &&
          (C / 64 * rs + 4) * rs < 65536 && rs * S < 65536 && out_ld >= 0 && (16 * out_ld + 64) * 2 < (int64_t(1) << 31) &&
-         ((M + 255) / 256) * ((pixels + 255) / 256) * images >= 240;
+         large_tiles_suit(M, pixels, C * rs, images, 1024);
 }
 
 int gemm_conv_large(int dtype, GemmArgs g, hipStream_t st) {

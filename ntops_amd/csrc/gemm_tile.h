@@ -543,6 +543,8 @@ int gemm_skinny_dma(int dtype, const GemmArgs& g, int j, hipStream_t st);
 // The 256 x 256 persistent kernel (gemm_large.hip): 16-bit products in the
 // matrix-core layouts (see run_gemm) that gemm_large_serves.
 bool gemm_large_serves(const GemmArgs& g);
+// Whether its tiles suit the product's size (k_min: see there).
+bool large_tiles_suit(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t k_min);
 int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipStream_t st);
 // Its channels-last convolution: k in 64-channel blocks; problems that
 // conv_large_serves (whatever the number of images in one launch).

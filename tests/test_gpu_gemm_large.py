@@ -80,3 +80,31 @@ def test_large_tiles_batch_and_full_c():
     exp = a.double() @ b.double()
     assert torch.equal(T.addmm(c, a, b), (exp + c.double()).float().to(dtype))
     assert torch.equal(T.addmm(c[:, :1], a, b), (exp + c[:, :1].double()).float().to(dtype))
+
+
+@pytest.mark.parametrize("m, n, k, layout, large", (
+    (2560, 3328, 512, "NN", True),     # 520 small tiles: past the two a CU holds
+    (2553, 3321, 512, "NT", True),     # the same, ragged
+    (2560, 3328, 520, "TN", True),
+    (2560, 3328, 504, "NT", False),    # too short for it
+    (2050, 4096, 2048, "NT", True),    # 544, the last row of large tiles nearly empty
+    (2050, 4096, 2040, "NN", False),
+    (2048, 4096, 1024, "NT", True),    # 512: one full round, K-major B
+    (2048, 4096, 1016, "NT", False),
+    (2048, 4096, 2048, "NN", True),    # N-major B from K = 2048
+    (2048, 4096, 2040, "NN", False),
+    (2048, 4096, 2048, "TN", False),   # M-major A
+    (1792, 4096, 2048, "NT", False),   # 448: seven eighths of a round, not past it
+    (384, 19456, 2048, "NT", False),   # 456, large tiles a quarter empty
+))
+def test_large_tiles_below_a_round(m, n, k, layout, large):
+    """Which products of fewer than 240 tiles take the kernel, and their sums (256 CUs)."""
+    dtype = torch.bfloat16
+    a, b, bias = ints(m, k, seed=11, dtype=dtype), ints(k, n, seed=12, dtype=dtype), ints(n, seed=13, dtype=dtype)
+    exp = a.double() @ b.double()
+    ag, bg = major(a, layout[0]), major(b, layout[1])
+    got = T.mm(ag, bg)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _lib.last_kernel().startswith("gemm_mfma 256x256" if large else "gemm_mfma 128x128"), _lib.last_kernel()
+    assert torch.equal(got, exp.float().to(dtype))
+    assert torch.equal(T.addmm(bias, ag, bg), (exp + bias.double()).float().to(dtype))
