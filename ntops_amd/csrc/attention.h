@@ -36,7 +36,8 @@ __device__ __forceinline__ int vslot(int r, int c) {
 
 // True when attn_decode serves this problem: 16-bit data whose head dim and
 // rows suit the matrix cores, no explicit mask, at most 16 query rows per key
-// / value head, and more than kDecodeMinKeys keys.
+// / value head, and more than kDecodeMinKeys keys -- or any but none, where
+// every CU gets a key / value head.
 bool attn_decode_serves(const AttnArgs& a);
 // Bytes of workspace with which attn_decode splits the keys over more blocks
 // (0: one block per key / value head is as good).

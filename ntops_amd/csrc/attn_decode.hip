@@ -421,9 +421,10 @@ int run_decode(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st) {
 bool attn_decode_serves(const AttnArgs& a) {
   const auto rows16 = [](const int64_t* s) { return s[3] == 1 && s[2] % 8 == 0 && s[1] % 8 == 0 && s[0] % 8 == 0; };
   const int64_t ld = std::max(a.ks[2], a.vs[2]);
-  return a.mask_dtype < 0 && decode_pays(static_cast<int64_t>(a.B) * a.Hkv, a.Skv) && static_cast<int64_t>(a.Sq) * (a.Hq / a.Hkv) <= 16 &&
-         a.D % 8 == 0 && a.D <= 128 && rows16(a.qs) && rows16(a.ks) && rows16(a.vs) && a.os[3] == 1 &&
-         a.os[2] % 4 == 0 && a.os[1] % 4 == 0 && a.os[0] % 4 == 0 && aligned16(a.q) && aligned16(a.k) &&
+  // (an empty cache has no tile to slice: the general kernel writes its zeros)
+  return a.mask_dtype < 0 && a.Skv > 0 && decode_pays(static_cast<int64_t>(a.B) * a.Hkv, a.Skv) &&
+         static_cast<int64_t>(a.Sq) * (a.Hq / a.Hkv) <= 16 && a.D % 8 == 0 && a.D <= 128 && rows16(a.qs) &&
+         rows16(a.ks) && rows16(a.vs) && a.os[3] == 1 && a.os[2] % 4 == 0 && a.os[1] % 4 == 0 && a.os[0] % 4 == 0 && aligned16(a.q) && aligned16(a.k) &&
          aligned16(a.v) && (reinterpret_cast<uintptr_t>(a.o) & 7u) == 0 && a.ks[2] >= a.D && a.vs[2] >= a.D &&
          (static_cast<int64_t>(a.Skv) + 64) * ld * 2 < 0x7fffffffLL &&
          static_cast<int64_t>(a.B) * a.Hkv <= 0x7fffffffLL / kDecodeMaxSplit;

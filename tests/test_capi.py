@@ -6,6 +6,8 @@ a message before any HIP call is made.  The torch wrappers refuse CPU tensors
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -149,3 +151,19 @@ def test_knobs_are_kept():
     torch.set_float32_matmul_precision("high")
     assert utils._get_matmul_input_precision() == InputPrecisionVariant.TF32
     torch.set_float32_matmul_precision("highest")
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="passes addresses that no GPU may follow")
+@pytest.mark.parametrize("b, heads, sq", ((1, 2, 1), (8, 32, 1), (16, 64, 16)))
+def test_sdpa_of_an_empty_cache_returns(b, heads, sq):
+    """No keys at all, few heads and at least one per CU: the call reaches its
+    launch (which fails here, without a GPU) instead of dividing by the keys.
+    In a process of its own, which a division by zero would end."""
+    code = (
+        "import ctypes; from ntops_amd import _lib; lib = _lib.load(); st = _lib.i64_array((64, 64, 64, 1));"
+        f"p = ctypes.c_void_p(1 << 20); rc = lib.ntops_sdpa(_lib.BF16, {b}, {heads}, {heads}, {sq}, 0, 64, p, st, p, st,"
+        "p, st, None, 0, None, 0, 0.125, p, st, None); print(rc, lib.ntops_last_kernel().decode());"
+        f"assert lib.ntops_sdpa_workspace(_lib.BF16, {b}, {heads}, {heads}, {sq}, 0, 64, 0) == 0")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stderr)
+    assert r.stdout.startswith("3 sdpa_fwd"), r.stdout

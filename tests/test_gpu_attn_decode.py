@@ -65,6 +65,27 @@ def test_decode(b, hq, hkv, sq, skv, d, causal, dtype):
     assert_close(out, oracle(q, k, v, causal), 1.6e-2, 1.6e-2, "unsplit")
 
 
+@pytest.mark.parametrize("b, h", ((1, 2), (8, 32)))
+@pytest.mark.parametrize("causal", (0, 2))
+def test_empty_cache(b, h, causal, monkeypatch):
+    """No keys: zeros, with few heads and with a head for every CU, through the
+    native host path, the Python one and the C ABI."""
+    q = torch.randn(b, h, 1, 64, device="cuda").bfloat16()
+    k = torch.empty(b, h, 0, 64, device="cuda").bfloat16()
+    args = dict(is_causal=causal > 0, causal_variant=CausalVariant.LOWER_RIGHT if causal else None)
+    assert (sdpa(q, k, k, **args) == 0).all()
+    assert _lib.last_kernel().startswith("sdpa_fwd"), _lib.last_kernel()
+    with monkeypatch.context() as mp:
+        mp.setattr(_lib, "fast", None)
+        assert (sdpa(q, k, k, **args) == 0).all()
+    out = torch.full_like(q, float("nan"))
+    st = lambda t: _lib.i64_array(t.stride())  # noqa: E731
+    _lib.check(_lib.load().ntops_sdpa(
+        _lib.BF16, b, h, h, 1, 0, 64, q.data_ptr(), st(q), None, st(k), None, st(k), None, 0, None, causal, 0.125,
+        out.data_ptr(), st(out), _lib.stream_of(out)), "sdpa")
+    assert (out == 0).all()
+
+
 def test_decode_special_values():
     """NaN and infinite scores, a causal row that sees no key, and a repeated
     call (bit for bit: the slices are combined in a fixed order)."""
