@@ -416,6 +416,14 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
   float m_i = neg_inf(), l_i = 0.f;  // reference max (base 2) of row my_q; this lane's half of its sum
   const float c = neg ? -a.scale_log2 : a.scale_log2;
+  // m_i is the rounded product max(S) c, which the fma's exact one misses by
+  // up to half an ulp: nothing near zero (2^-15 of P's exponent at 2^10), but
+  // 64 at the 1e10 of a row that a large finite mask value closes, which took
+  // P to 0 or past f16.  From kFarMax on the scores are rounded like m_i, so
+  // that the largest P is exactly 1.  ((8, 16, 1000, 64) f16 bool 60.8 us
+  // without the test, 61.2 with it.)
+  constexpr float kFarMax = 1024.f;
+  bool far = false;  // some row of the wave is there
   // last key of row my_q, relative to this lane's column group
   int lim = a.Skv - 1;
   if (a.causal) lim = min(lim, my_q + off);
@@ -493,13 +501,21 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+      far = __any(fabsf(m_i) >= kFarMax && m_i > neg_inf());
     }
     const float mb = m_i == neg_inf() ? 0.f : m_i;  // fully masked so far: P = 0
     float x[2][16];
+    if (far) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(fmaf(s[t][e], c, -mb));
+        for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(add_nc(mul_nc(s[t][e], c), -mb));
+    } else {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(fmaf(s[t][e], c, -mb));
+    }
     {
       float r[16];
 #pragma unroll

@@ -67,3 +67,43 @@ def test_scale_signs(scale, masked):
     got = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=None if mask is None else mask.cuda(), scale=scale)
     exp = oracle(q, k, v, None if mask is None else mask.expand(1, 2, 20, 150), scale)
     assert_close(got, exp, 1.6e-2, 1.6e-2, f"scale {scale}")
+
+
+# the large finite values that programs close keys with; tiles of 64 keys
+@pytest.mark.parametrize("value", (-65504.0, -1e6, -1e9, -1e10, -1e30))
+@pytest.mark.parametrize("mask_dtype", (torch.float16, torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("d", (64, 80, 128))
+def test_large_finite_mask_values(value, mask_dtype, dtype, d):
+    """Rows whose first or middle tile is closed by a finite value are as if it
+    were closed altogether (exp(-65504 + a few tens) is 0 in 64 bits too).  A
+    row closed throughout has all its scores at the value: with a zero query
+    they are equal, so the row is the mean of V; with any other the values are
+    too coarse for the scores (half a unit and more from 1e6 on), but P still
+    sums to 1 and the row lies among V's."""
+    if mask_dtype == torch.float16 and value < -65504:
+        pytest.skip("not a finite value of the type")
+    g = torch.Generator().manual_seed(d)
+    b, h, sq, skv = 2, 2, 72, 200
+    q, k, v = (torch.randn(b, h, s, d, generator=g).to(dtype) for s in (sq, skv, skv))
+    mask = torch.zeros(b, 1, sq, skv)
+    mask[:, :, 0:24, :64] = value      # left padding of a tile
+    mask[:, :, 24:40, 64:128] = value  # a tile in the middle
+    mask[:, :, 20:32, 192:] = value    # the last, partial one
+    mask[:, :, 56:] = value            # rows closed throughout
+    q[:, :, 56:64] = 0
+    mask = mask.to(mask_dtype)
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), attn_mask=mask.cuda()).cpu()
+    assert _lib.last_kernel().startswith("sdpa_fwd"), _lib.last_kernel()
+    exp = oracle(q, k, v, mask.expand(b, h, sq, skv))
+    assert_close(got[:, :, :56], exp[:, :, :56], 1.6e-2, 1.6e-2, "some tiles closed")
+    mean = v.double().mean(2, keepdim=True)
+    # the sum of 200 equal P is exact and so is each P V product; what is left
+    # is the fp32 sums (far below) and one rounding of the result
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert_close(got[:, :, 56:64], mean.expand(b, h, 8, d), ulp, 1e-5, "equal scores")
+    # P is rounded (half an ulp of it each way), its sum is not
+    lo, hi = v.amin(2, keepdim=True).double(), v.amax(2, keepdim=True).double()
+    slack = 2 * ulp * v.abs().amax().double()
+    rest = got[:, :, 64:].double()
+    assert ((rest >= lo - slack) & (rest <= hi + slack)).all()
