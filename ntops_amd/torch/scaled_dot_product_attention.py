@@ -24,9 +24,10 @@ _MASK_DTYPES = (torch.bool, torch.float32, torch.float16, torch.bfloat16)
 
 def _write_slots(key, key_slot, value, value_slot):
     """key_slot[...] = key and value_slot[...] = value; one launch for a pair
-    of plain copies (the usual case), else a cast kernel each."""
-    shape, dtype = key.shape, key.dtype
-    if all(t.shape == shape and t.dtype == dtype for t in (key_slot, value, value_slot)):
+    of plain copies on one device (the usual case), else a cast kernel each,
+    which refuses a slot that is not on a GPU."""
+    shape, dtype, device = key.shape, key.dtype, key.device
+    if all(t.shape == shape and t.dtype == dtype and t.device == device for t in (key_slot, value, value_slot)):
         rc = _lib.load().ntops_copy2(
             _lib.dtype_code(dtype), len(shape), _lib.i64_array(shape),
             key.data_ptr(), _strides(key), key_slot.data_ptr(), _strides(key_slot),

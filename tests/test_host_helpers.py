@@ -124,3 +124,35 @@ def test_rows_of_reads_row_views_in_place():
         assert rs == 1024 and copied
     finally:
         U._contiguous = real
+
+
+def test_cache_slots_on_another_device_are_not_copied_blindly(monkeypatch):
+    """A key or value slot that is not on the operands' device takes the cast
+    path, which asks for the slot's own stream and so refuses host memory; the
+    two-copy launch gets four tensors of one device only."""
+    import importlib
+
+    from ntops_amd import _lib
+
+    S = importlib.import_module("ntops_amd.torch.scaled_dot_product_attention")
+    calls = []
+
+    class Lib:
+        @staticmethod
+        def ntops_copy2(*_):
+            calls.append("copy2")
+            return 0
+
+    monkeypatch.setattr(_lib, "load", lambda: Lib)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: None)
+    monkeypatch.setattr(S, "_cast_into", lambda src, dst: calls.append("cast"))
+    here, host = (torch.zeros(2, 3, device=d) for d in ("meta", "cpu"))
+    S._write_slots(here, here, here, here)
+    assert calls == ["copy2"]
+    for key_slot, value_slot in ((host, here), (here, host), (host, host)):
+        calls.clear()
+        S._write_slots(here, key_slot, here, value_slot)
+        assert calls == ["cast", "cast"]
+    monkeypatch.undo()
+    with pytest.raises((TypeError, RuntimeError)):
+        _lib.stream_of(host)
