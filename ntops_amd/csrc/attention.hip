@@ -185,6 +185,16 @@ struct KvDma {
   }
 };
 
+// 0 * x of 8 16-bit values: NaN where x is not finite.
+template <typename T>
+__device__ __forceinline__ u32x4 times_zero(u32x4 x) {
+  constexpr uint32_t kExp = std::is_same<T, __bf16>::value ? 0x7f80u : 0x7c00u;
+  const auto word = [](uint32_t w) {
+    return ((w & kExp) == kExp ? 0x7fffu : 0u) | ((w >> 16 & kExp) == kExp ? 0x7fff0000u : 0u);
+  };
+  return u32x4{word(x.x), word(x.y), word(x.z), word(x.w)};
+}
+
 // MM: explicit-mask mode -- 0 none, 1 / 2 the last, partial tile by runs of 4
 // keys (rows 4-element aligned) / by elements; ESZ: mask element bytes (1 bool, 2
 // fp16 / bf16, 4 fp32).  Both are template parameters so that every mask
@@ -225,8 +235,14 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       qf[ks] = u32x4{0, 0, 0, 0};
   }
   // a negative scale: -Q under its magnitude, so that the max of the scaled
-  // scores is the scaled max (a zero scale takes the generic kernel)
+  // scores is the scaled max; a zero scale (MM = 0 only): 0 Q under one, so
+  // that a key without a score stays at -inf
   const bool neg = a.scale_log2 < 0.f;
+  const bool zero = a.scale_log2 == 0.f;
+  if (zero) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = times_zero<T>(qf[ks]);
+  }
   if (neg) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] ^= 0x80008000u;
@@ -415,7 +431,7 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
   float m_i = neg_inf(), l_i = 0.f;  // reference max (base 2) of row my_q; this lane's half of its sum
-  const float c = neg ? -a.scale_log2 : a.scale_log2;
+  const float c = zero ? 1.f : neg ? -a.scale_log2 : a.scale_log2;
   // m_i is the rounded product max(S) c, which the fma's exact one misses by
   // up to half an ulp: nothing near zero (2^-15 of P's exponent at 2^10), but
   // 64 at the 1e10 of a row that a large finite mask value closes, which took
@@ -1300,7 +1316,7 @@ int run_attention(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st)
     const bool mask_fits = a.mask_dtype < 0 ||
                            (a.ms[3] == 1 && a.scale_log2 != 0.f &&
                             (static_cast<int64_t>(a.Sq) * a.ms[2] + a.Skv + 68) * esz < 0x7fffffffLL);
-    if (mfma && mask_fits && (a.scale_log2 > 0.f || a.scale_log2 < 0.f)) {
+    if (mfma && mask_fits && a.scale_log2 == a.scale_log2) {
       const int nqb = (a.Sq + 127) / 128;
       const int64_t total = static_cast<int64_t>(nqb) * a.Hq * a.B;
       if (total > 0x7fffffffLL) return set_error(NTOPS_ERR_UNSUPPORTED, "sdpa: too many blocks");

@@ -107,3 +107,28 @@ def test_large_finite_mask_values(value, mask_dtype, dtype, d):
     slack = 2 * ulp * v.abs().amax().double()
     rest = got[:, :, 64:].double()
     assert ((rest >= lo - slack) & (rest <= hi + slack)).all()
+
+
+@pytest.mark.parametrize("sq, skv, d, causal", ((20, 150, 128, 0), (300, 190, 64, 2), (190, 300, 80, 1)))
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+def test_zero_scale_stays_on_the_matrix_cores(sq, skv, d, causal, dtype):
+    """A zero scale without a mask: equal scores over the keys a row sees, none
+    for a row that sees no key, NaN where a query or key is not finite."""
+    g = torch.Generator().manual_seed(sq)
+    q, k, v = (torch.randn(1, 2, s, d, generator=g).to(dtype) for s in (sq, skv, skv))
+    args = dict(scale=0.0, is_causal=causal > 0, causal_variant=causal or None)
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), **args)
+    assert _lib.last_kernel().startswith("sdpa_fwd"), _lib.last_kernel()
+    i, j = torch.arange(sq)[:, None], torch.arange(skv)[None]
+    seen = (j <= i + (skv - sq if causal == 2 else 0)) if causal else torch.ones(sq, skv, dtype=torch.bool)
+    p = seen.double() / seen.sum(1, keepdim=True).clamp_min(1)
+    # P = 1 exactly: the fp32 sums and one rounding of the result
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert_close(got, p @ v.double(), ulp, 1e-5, "zero scale")
+    q[0, 0, 7, 5] = float("-inf")
+    k[0, 1, skv // 2, 3] = float("nan")
+    bad = sdpa(q.cuda(), k.cuda(), v.cuda(), **args).cpu()
+    rows = torch.zeros(1, 2, sq, dtype=torch.bool)
+    rows[0, 0, 7] = seen[7].any()
+    rows[0, 1] = seen[:, skv // 2]
+    assert bad[rows].isnan().all() and torch.equal(bad[~rows], got.cpu()[~rows])
