@@ -115,6 +115,20 @@ PyObject* wrap2(const at::Tensor& a, const at::Tensor& b) {
 }
 PyObject* none() { Py_RETURN_NONE; }
 
+// The interpreter is free while a call allocates and launches (either may wait
+// for the device), as it is in torch's own allocations and in ctypes calls;
+// no Python object is touched inside.
+class NoGil {
+ public:
+  NoGil() : state_(PyEval_SaveThread()) {}
+  ~NoGil() { PyEval_RestoreThread(state_); }
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 // A Python float or int (not a bool) as a double.
 bool number(PyObject* o, double& v) {
   if (PyFloat_CheckExact(o)) {
@@ -194,12 +208,16 @@ PyObject* unary(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* st;
   if (!x || code16_32(*x) < 0 || !x->is_contiguous() || x->dim() > 16 || !current(dev, st) || x->get_device() != dev)
     return none();
-  at::Tensor y = at::empty_like(*x);
-  const auto xs = x->strides(), ys = y.strides();
-  if (f_unary(static_cast<int>(PyLong_AsLong(a[0])), code16_32(*x), static_cast<int>(x->dim()), x->sizes().data(),
-              x->data_ptr(), xs.data(), y.data_ptr(), ys.data(), st) != NTOPS_OK)
-    return none();
-  return wrap(y);
+  const int op = static_cast<int>(PyLong_AsLong(a[0]));
+  at::Tensor y;
+  int rc;
+  {
+    NoGil free;
+    y = at::empty_like(*x);
+    rc = f_unary(op, code16_32(*x), static_cast<int>(x->dim()), x->sizes().data(), x->data_ptr(), x->strides().data(),
+                 y.data_ptr(), y.strides().data(), st);
+  }
+  return rc == NTOPS_OK ? wrap(y) : none();
   NTOPS_END
 }
 
@@ -224,11 +242,14 @@ PyObject* softmax(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (int64_t i = dim + 1; i < x->dim(); ++i) inner *= x->size(i);
   const int64_t size = x->size(dim);
   const int64_t strides[3] = {size * inner, inner, 1};
-  at::Tensor y = new_like(*x, x->sizes());
-  if (f_softmax(code16_32(*x), code16_32(*x), outer, size, inner, x->data_ptr(), strides, y.data_ptr(), strides, st) !=
-      NTOPS_OK)
-    return none();
-  return wrap(y);
+  at::Tensor y;
+  int rc;
+  {
+    NoGil free;
+    y = new_like(*x, x->sizes());
+    rc = f_softmax(code16_32(*x), code16_32(*x), outer, size, inner, x->data_ptr(), strides, y.data_ptr(), strides, st);
+  }
+  return rc == NTOPS_OK ? wrap(y) : none();
   NTOPS_END
 }
 
@@ -246,11 +267,15 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   const int64_t cols = norm_cols(*x, a[1]);
   if (cols <= 0 || !norm_param(a[2], *x, cols, static_cast<int>(dev), w)) return none();
-  at::Tensor y = new_like(*x, x->sizes());
-  if (f_rms_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, w ? w->data_ptr() : nullptr, 0,
-                 w ? code16_32(*w) : code16_32(*x), eps, y.data_ptr(), cols, st) != NTOPS_OK)
-    return none();
-  return wrap(y);
+  at::Tensor y;
+  int rc;
+  {
+    NoGil free;
+    y = new_like(*x, x->sizes());
+    rc = f_rms_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, w ? w->data_ptr() : nullptr, 0,
+                    w ? code16_32(*w) : code16_32(*x), eps, y.data_ptr(), cols, st);
+  }
+  return rc == NTOPS_OK ? wrap(y) : none();
   NTOPS_END
 }
 
@@ -276,11 +301,15 @@ PyObject* layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (w && b->scalar_type() != w->scalar_type()) return none();
     code = code16_32(*b);
   }
-  at::Tensor y = new_like(*x, x->sizes());
-  if (f_layer_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, w ? w->data_ptr() : nullptr,
-                   b ? b->data_ptr() : nullptr, 0, code, eps, y.data_ptr(), cols, st) != NTOPS_OK)
-    return none();
-  return wrap(y);
+  at::Tensor y;
+  int rc;
+  {
+    NoGil free;
+    y = new_like(*x, x->sizes());
+    rc = f_layer_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, w ? w->data_ptr() : nullptr,
+                      b ? b->data_ptr() : nullptr, 0, code, eps, y.data_ptr(), cols, st);
+  }
+  return rc == NTOPS_OK ? wrap(y) : none();
   NTOPS_END
 }
 
@@ -299,12 +328,17 @@ PyObject* add_rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return none();
   const int64_t cols = norm_cols(*x, a[2]);
   if (cols <= 0 || !norm_param(a[3], *x, cols, static_cast<int>(dev), w)) return none();
-  at::Tensor y = new_like(*x, x->sizes()), h = new_like(*x, x->sizes());
-  if (f_add_rms_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, r->data_ptr(), cols,
-                     w ? w->data_ptr() : nullptr, 0, w ? code16_32(*w) : code16_32(*x), eps, y.data_ptr(), cols,
-                     h.data_ptr(), cols, st) != NTOPS_OK)
-    return none();
-  return wrap2(y, h);
+  at::Tensor y, h;
+  int rc;
+  {
+    NoGil free;
+    y = new_like(*x, x->sizes());
+    h = new_like(*x, x->sizes());
+    rc = f_add_rms_norm(code16_32(*x), x->numel() / cols, cols, x->data_ptr(), cols, r->data_ptr(), cols,
+                        w ? w->data_ptr() : nullptr, 0, w ? code16_32(*w) : code16_32(*x), eps, y.data_ptr(), cols,
+                        h.data_ptr(), cols, st);
+  }
+  return rc == NTOPS_OK ? wrap2(y, h) : none();
   NTOPS_END
 }
 
@@ -328,12 +362,18 @@ PyObject* rope_qk(PyObject*, PyObject* const* a, Py_ssize_t n) {
       cs.size(0) < S || (tw != D && tw != D / 2) || cs.size(1) != tw || sn.stride(1) != 1 || cs.stride(1) != 1 ||
       sn.stride(0) != cs.stride(0))
     return none();
-  at::Tensor qo = at::empty_like(q), ko = at::empty_like(k);
-  if (f_rope_qk(code16_32(q), B, S, q.size(2), k.size(2), D, q.data_ptr(), q.strides().data(), k.data_ptr(),
-                k.strides().data(), sn.data_ptr(), cs.data_ptr(), sn.stride(0), tw, a[4] == Py_True ? 1 : 0,
-                qo.data_ptr(), qo.strides().data(), ko.data_ptr(), ko.strides().data(), st) != NTOPS_OK)
-    return none();
-  return wrap2(qo, ko);
+  const int interleaved = a[4] == Py_True ? 1 : 0;
+  at::Tensor qo, ko;
+  int rc;
+  {
+    NoGil free;
+    qo = at::empty_like(q);
+    ko = at::empty_like(k);
+    rc = f_rope_qk(code16_32(q), B, S, q.size(2), k.size(2), D, q.data_ptr(), q.strides().data(), k.data_ptr(),
+                   k.strides().data(), sn.data_ptr(), cs.data_ptr(), sn.stride(0), tw, interleaved, qo.data_ptr(),
+                   qo.strides().data(), ko.data_ptr(), ko.strides().data(), st);
+  }
+  return rc == NTOPS_OK ? wrap2(qo, ko) : none();
   NTOPS_END
 }
 
@@ -361,17 +401,20 @@ PyObject* gemm(const at::Tensor* c, PyObject* pa, PyObject* pb, double beta, dou
     cst[2] = cn == 1 && N != 1 ? 0 : c->stride(c->dim() - 1);
     cst[1] = cm == 1 && M != 1 ? 0 : c->dim() == 2 ? c->stride(0) : 0;
   }
-  at::Tensor out = new_like(*x, {M, N});
   const int code = code16_32(*x);
-  const int64_t bytes = f_gemm_workspace(code, 1, M, N, K);
-  at::Tensor ws;
-  if (bytes > 0) ws = workspace(*x, bytes);
   const int64_t ast[3] = {0, x->stride(0), 1}, bst[3] = {0, w->stride(0), w->stride(1)}, dst[3] = {0, N, 1};
-  if (f_gemm_ws(code, 1, M, N, K, x->data_ptr(), ast, w->data_ptr(), bst, c ? c->data_ptr() : nullptr,
-                c ? cst : nullptr, alpha, beta, out.data_ptr(), dst, bytes > 0 ? ws.data_ptr() : nullptr, bytes, st) !=
-      NTOPS_OK)
-    return none();
-  return wrap(out);
+  at::Tensor out;
+  int rc;
+  {
+    NoGil free;
+    out = new_like(*x, {M, N});
+    const int64_t bytes = f_gemm_workspace(code, 1, M, N, K);
+    at::Tensor ws;
+    if (bytes > 0) ws = workspace(*x, bytes);
+    rc = f_gemm_ws(code, 1, M, N, K, x->data_ptr(), ast, w->data_ptr(), bst, c ? c->data_ptr() : nullptr,
+                   c ? cst : nullptr, alpha, beta, out.data_ptr(), dst, bytes > 0 ? ws.data_ptr() : nullptr, bytes, st);
+  }
+  return rc == NTOPS_OK ? wrap(out) : none();
 }
 PyObject* mm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   NTOPS_TRY
@@ -425,30 +468,36 @@ PyObject* sdpa(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
   }
   const int causal = static_cast<int>(PyLong_AsLong(a[4]));
+  const at::Tensor* p[4] = {};
   if (a[7] != Py_None) {
-    const at::Tensor* p[4];
     for (int i = 0; i < 4; ++i) {  // key, value, key slot, value slot
       p[i] = plain(a[7 + i]);
       if (!p[i] || p[i]->get_device() != dev || p[i]->scalar_type() != p[0]->scalar_type() || p[i]->dim() > 16 ||
           code16_32(*p[i]) < 0 || p[i]->sizes() != p[0]->sizes())
         return none();
     }
-    if (f_copy2(code16_32(*p[0]), static_cast<int>(p[0]->dim()), p[0]->sizes().data(), p[0]->data_ptr(),
-                p[0]->strides().data(), p[2]->data_ptr(), p[2]->strides().data(), p[1]->data_ptr(),
-                p[1]->strides().data(), p[3]->data_ptr(), p[3]->strides().data(), st) != NTOPS_OK)
-      return none();
   }
-  at::Tensor out = new_like(*q, q->sizes());
   const int code = code16_32(*q);
-  int64_t bytes = 0;
-  at::Tensor ws;
-  if (!m && Sq <= 16) bytes = f_sdpa_workspace(code, B, Hq, Hk, Sq, Sk, D, 0);
-  if (bytes > 0) ws = workspace(*q, bytes);
-  if (f_sdpa_ws(code, B, Hq, Hk, Sq, Sk, D, q->data_ptr(), q->strides().data(), k->data_ptr(), k->strides().data(),
-                v->data_ptr(), v->strides().data(), m ? m->data_ptr() : nullptr, mcode, m ? mst : nullptr, causal, scale,
-                out.data_ptr(), out.strides().data(), bytes > 0 ? ws.data_ptr() : nullptr, bytes, st) != NTOPS_OK)
-    return none();
-  return wrap(out);
+  at::Tensor out;
+  int rc = NTOPS_OK;
+  {
+    NoGil free;
+    if (p[0])
+      rc = f_copy2(code16_32(*p[0]), static_cast<int>(p[0]->dim()), p[0]->sizes().data(), p[0]->data_ptr(),
+                   p[0]->strides().data(), p[2]->data_ptr(), p[2]->strides().data(), p[1]->data_ptr(),
+                   p[1]->strides().data(), p[3]->data_ptr(), p[3]->strides().data(), st);
+    if (rc == NTOPS_OK) {
+      out = new_like(*q, q->sizes());
+      int64_t bytes = 0;
+      at::Tensor ws;
+      if (!m && Sq <= 16) bytes = f_sdpa_workspace(code, B, Hq, Hk, Sq, Sk, D, 0);
+      if (bytes > 0) ws = workspace(*q, bytes);
+      rc = f_sdpa_ws(code, B, Hq, Hk, Sq, Sk, D, q->data_ptr(), q->strides().data(), k->data_ptr(), k->strides().data(),
+                     v->data_ptr(), v->strides().data(), m ? m->data_ptr() : nullptr, mcode, m ? mst : nullptr, causal,
+                     scale, out.data_ptr(), out.strides().data(), bytes > 0 ? ws.data_ptr() : nullptr, bytes, st);
+    }
+  }
+  return rc == NTOPS_OK ? wrap(out) : none();
   NTOPS_END
 }
 

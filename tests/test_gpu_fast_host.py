@@ -2,7 +2,9 @@
 bit for bit over the forms each op accepts, the same errors for those it
 refuses, and None (the Python path) for tensors that are not plain."""
 
+import ctypes
 import itertools
+from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
@@ -137,3 +139,56 @@ def test_native_and_python_paths_agree(monkeypatch):
         z = T.silu(y)
     s.synchronize()
     assert torch.equal(z, T.silu(T.silu(big)))
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_native_calls_free_the_interpreter():
+    """Each op with the library's entry points replaced by PyGILState_Check,
+    which returns 0 (NTOPS_OK, so the op returns its output) where the calling
+    thread has let the interpreter go and 1 (so it returns None) where not."""
+    lib = _lib.load()
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    x, w = torch.randn(4, 64, device="cuda"), torch.randn(64, 64, device="cuda")
+    q = torch.randn(1, 2, 4, 64, device="cuda")
+    f = _lib.fast
+    assert f.init(dict.fromkeys(_lib.EXPORTED, check), torch._C._cuda_getDevice, _lib._raw_stream)
+    try:
+        got = {
+            "unary": f.unary(1, x), "softmax": f.softmax(x, -1), "rms_norm": f.rms_norm(x, (64,), None, 1e-6),
+            "layer_norm": f.layer_norm(x, (64,), None, None, 1e-5),
+            "add_rms_norm": f.add_rms_norm(x, x, (64,), None, 1e-6), "rope_qk": f.rope_qk(q, q, w, w, True),
+            "mm": f.mm(x, w), "addmm": f.addmm(x, x, w, 1, 1),
+            "sdpa": f.sdpa(q, q, q, None, 0, None, False, None, None, None, None),
+            "sdpa slots": f.sdpa(q, q, q, None, 0, None, False, q, q, q, q),
+        }
+    finally:
+        _lib._init_fast(lib)
+    assert not [name for name, r in got.items() if r is None]
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_native_calls_from_several_threads():
+    """Four threads, each on a stream of its own, through calls that allocate
+    outputs and workspaces: every result equals the one computed alone."""
+    ins = [(torch.randn(40, 4096, device="cuda").bfloat16(), torch.randn(1024, 4096, device="cuda").bfloat16(),
+            torch.randn(1, 8, 1, 64, device="cuda").half(), torch.randn(1, 2, 2048, 64, device="cuda").half())
+           for _ in range(4)]
+
+    def step(x, w, q, kv):
+        return (T.mm(T.silu(T.rms_norm(x, (4096,))), w.t()),
+                T.scaled_dot_product_attention(q, kv, kv, enable_gqa=True))
+
+    alone = [step(*i) for i in ins]
+    torch.cuda.synchronize()
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            outs = [step(*ins[i]) for _ in range(50)]
+        stream.synchronize()
+        return all(torch.equal(a, b) for o in outs for a, b in zip(o, alone[i]))
+
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(work, range(4)))
