@@ -167,3 +167,17 @@ def test_sdpa_of_an_empty_cache_returns(b, heads, sq):
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stderr)
     assert r.stdout.startswith("3 sdpa_fwd"), r.stdout
+
+
+def test_library_builds_without_torch(tmp_path):
+    """The make plan for a Python that has no torch: the library as always,
+    the wrappers' extension left out."""
+    make = ["make", "-n", "-B", "-C", os.path.join(ROOT, "ntops_amd", "csrc")]
+    bare = tmp_path / "python"
+    bare.write_text(f"#!/bin/sh\nexec {sys.executable} -S -E \"$@\"\n")
+    bare.chmod(0o755)
+    for python, built in ((sys.executable, True), (str(bare), False), (str(tmp_path / "none"), False)):
+        r = subprocess.run([*make, f"PYTHON={python}"], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        assert "libntops_amd.so" in r.stdout and "capi.hip" in r.stdout
+        assert ("host/fast.cpp -o" in r.stdout) == built, python
