@@ -1348,15 +1348,12 @@ int pick_tile(const GemmArgs& g, hipStream_t st) {
   // ones at K = 1600, 6 to 14 % faster at 4096 and above; M-major A not taken)
   const int64_t k_min = !AK ? INT64_MAX : BKM ? 1024 : 2048;
   if (g.K > 256 && (big_tiles >= 240 || (large_tiles_suit(g.M, g.N, g.K, g.batch, k_min) && gemm_large_serves(g)))) {
-    const bool even = g.M % 256 == 0 && g.N % 256 == 0 && g.K % kBK == 0;
     // the persistent kernel: no C or a bias row, any output layout and edges
-    if (gemm_large_serves(g)) {
-      const int64_t interior = static_cast<int64_t>(g.M / 256) * (g.N / 256) * g.batch;
-      note_kernel("gemm_mfma 256x256 s4 %s %s %s", AK ? "A:K" : "A:M", BKM ? "B:K" : "B:N",
-                  even ? "even" : g.K % kBK == 0 && interior >= 240 ? "even+edges" : "ragged");
+    if (gemm_large_serves(g))
       return gemm_large(std::is_same<T, __bf16>::value ? NTOPS_BF16 : NTOPS_F16, AK, BKM, g, st);
-    }
-    if (even) return launch_mfma<T, 256, 256, 2, 4, kBK, kStages, AK, BKM, true>(g, st);
+    // a C with a value per row or element
+    if (g.M % 256 == 0 && g.N % 256 == 0 && g.K % kBK == 0)
+      return launch_mfma<T, 256, 256, 2, 4, kBK, kStages, AK, BKM, true>(g, st);
     // M or N not a multiple of 256: the bounds-checked kernel runs a third
     // slower than the even one over the whole product (bf16 8192 x 50264 x
     // 768: 839 against 625 us at N = 50176), so the even kernel takes the

@@ -646,6 +646,7 @@ bool gemm_large_serves(const GemmArgs& g) {
 }
 
 int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipStream_t st) {
+  note_kernel("gemm_large %s %s", a_kmajor ? "A:K" : "A:M", b_kmajor ? "B:K" : "B:N");
   return dtype == NTOPS_BF16 ? run_large<__bf16>(a_kmajor, b_kmajor, g, st)
                              : run_large<_Float16>(a_kmajor, b_kmajor, g, st);
 }
@@ -694,7 +695,7 @@ int gemm_conv_large(int dtype, GemmArgs g, hipStream_t st) {
   g.cl_mq = static_cast<uint32_t>(((uint64_t(1) << 32) + g.cl_q - 1) / g.cl_q);
   g.cl_mrs = (65536u + g.cv_rs - 1) / g.cv_rs;
   g.cl_ms = (65536u + g.cv_s - 1) / g.cv_s;
-  note_kernel("gemm_mfma 256x256 s4 A:K B:K %s conv_cl", g.M % 256 == 0 && g.N % 256 == 0 ? "even" : "ragged");
+  note_kernel("gemm_large A:K B:K conv_cl");
   return dtype == NTOPS_BF16 ? run_conv_large<__bf16>(g, st) : run_conv_large<_Float16>(g, st);
 }
 

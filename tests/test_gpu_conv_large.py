@@ -44,8 +44,7 @@ def test_conv_large(case, dtype):
     wt = small_ints(g, k, c, r, s).to(dtype)
     b = small_ints(g, k).to(dtype) if has_bias else None
     got = conv2d(x.cuda(), wt.cuda(), b if b is None else b.cuda(), stride=stride, padding=pad, dilation=dil)
-    kern = _lib.last_kernel()
-    assert kern.startswith("gemm_mfma 256x256") and kern.endswith("conv_cl"), kern
+    assert _lib.last_kernel() == "gemm_large A:K B:K conv_cl", _lib.last_kernel()
     for img in sorted({0, n // 2, n - 1}):
         exp = exact_image(x[img], wt, b, stride, pad, dil, *got.shape[2:])
         assert torch.equal(got[img].cpu(), exp.to(dtype)), f"image {img}"
@@ -62,6 +61,7 @@ def test_conv_large_bias_forms_and_chunks():
     xg, wg, bg = x.cuda(), wt.cuda(), bias.cuda()
     exp = {img: exact_image(x[img], wt, bias[::2], 1, 1, 1, h, h).bfloat16() for img in (0, 119, 120, 239, 240)}
     got = conv2d(xg, wg, bg[::2], padding=1)
+    assert _lib.last_kernel() == "gemm_mfma 256x256 s4 A:K B:K even conv_cl", _lib.last_kernel()
     out = torch.full((n, k, h, h), float("nan"), dtype=torch.bfloat16, device="cuda")
     lib = _lib.load()
     geo = (c, h, h, k, 3, 3, h, h, 1, 1, 1, 1, 1, 1)
@@ -72,6 +72,7 @@ def test_conv_large_bias_forms_and_chunks():
     rc = lib.ntops_conv2d(_lib.BF16, n, *geo, xg.data_ptr(), st(xg), wg.data_ptr(), st(wg), even.data_ptr(), 1,
                           out.data_ptr(), st(out), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
     assert rc == 0, lib.ntops_last_error()
+    assert _lib.last_kernel() == "gemm_large A:K B:K conv_cl", _lib.last_kernel()
     for img, e in exp.items():
         assert torch.equal(got[img].cpu(), e), f"strided bias, image {img}"
         assert torch.equal(out[img].cpu(), e), f"chunks, image {img}"

@@ -75,7 +75,7 @@ def expected16(m, n, k, layout, batch=1):
     if k <= 128 and m % 128 == 0 and n % 128 == 0:
         return "gemm_panel "
     if -(-m // 256) * -(-n // 256) * batch >= 240 and k > 256:
-        return "gemm_mfma 256x256 "
+        return "gemm_large "
     return "gemm_mfma 128x128 "
 
 
@@ -113,7 +113,7 @@ def test_mm_layouts(m, n, k, dtype, layout):
     check(got, a, b, dtype, what=f"mm {layout}")
 
 
-# The 256 x 256 tile kernel (>= 240 tiles, K > 256): every instantiation --
+# The persistent 256 x 256 tile kernel (>= 240 tiles, K > 256): every instantiation --
 # bf16 and fp16, K-major or M-major A, N-major or K-major B, even edges
 # (M, N multiples of 256, K of 32) and ragged ones (all three off that grid;
 # multiples of 8 so that every layout qualifies) -- each as mm and as addmm
@@ -132,8 +132,7 @@ def test_mm_256_tiles(dtype, layout, edges):
     bias = torch.randn(n, generator=g).to(dtype)
     ag = a.cuda() if layout[0] == "N" else a.t().contiguous().cuda().t()
     bg = b.cuda() if layout[1] == "N" else b.t().contiguous().cuda().t()
-    kernel = (f"gemm_mfma 256x256 s4 {'A:K' if layout[0] == 'N' else 'A:M'} "
-              f"{'B:N' if layout[1] == 'N' else 'B:K'} {edges}")
+    kernel = f"gemm_large {'A:K' if layout[0] == 'N' else 'A:M'} {'B:N' if layout[1] == 'N' else 'B:K'}"
     got = ntops_amd.torch.mm(ag, bg)
     assert _lib.last_kernel() == kernel
     check(got, a, b, dtype, what=f"mm 256 {layout} {edges}")
@@ -237,80 +236,110 @@ def test_gemm_ragged_output_through_the_c_abi(m, n, k, dtype, form):
           what=f"ragged output {form}")
 
 
+def c_gemm(a, b, c, c_strides, out, out_strides, alpha=1.0, beta=1.0):
+    """ntops_gemm on (batch, m, k) a and (batch, k, n) b, C and out of any strides."""
+    (bsz, m, k), n = a.shape, b.shape[2]
+    rc = _lib.load().ntops_gemm(
+        _lib.dtype_code(a.dtype), bsz, m, n, k, a.data_ptr(), _lib.i64_array(a.stride()), b.data_ptr(),
+        _lib.i64_array(b.stride()), c.data_ptr(), _lib.i64_array(c_strides), alpha, beta, out.data_ptr(),
+        _lib.i64_array(out_strides), _lib.stream_of(out))
+    _lib.check(rc, "ntops_gemm")
+
+
+@pytest.mark.parametrize("form", ("full", "column"))
 @pytest.mark.parametrize("m, n, k, b_kmajor", [(4100, 4200, 512, False), (4100, 4200, 512, True),
                                               (4136, 4099, 320, True), (4096, 4360, 1024, False)])
-def test_mm_even_interior_and_edge_strips(m, n, k, b_kmajor):
-    """Large products whose M or N is not a multiple of 256: the even 256 x
-    256 kernel on the interior, ragged 128 x 128 tiles on the right and bottom
-    strips.  Small-integer operands make every fp32 sum exact, so each output
-    equals the double-precision product rounded once to bf16; an addmm with a
-    bias row is checked on sampled rows against the oracle."""
+def test_addmm_even_interior_and_edge_strips(m, n, k, b_kmajor, form):
+    """Large products whose M or N is not a multiple of 256, under a C with a
+    value per element or per row (without one the persistent kernel serves
+    them): the even 256 x 256 kernel on the interior, ragged 128 x 128 tiles on
+    the right and bottom strips.  Small-integer operands make every fp32 sum
+    exact, so each output equals the double-precision product rounded once to
+    bf16; random operands are checked on sampled rows against the oracle."""
     g = torch.Generator().manual_seed(m + n + k)
+    cn = n if form == "full" else 1
     a = torch.randint(-8, 9, (m, k), generator=g).to(torch.bfloat16)
     b = torch.randint(-8, 9, (k, n), generator=g).to(torch.bfloat16)
+    c = torch.randint(-8, 9, (m, cn), generator=g).to(torch.bfloat16)
     bg = b.cuda() if not b_kmajor else b.t().contiguous().cuda().t()
-    got = ntops_amd.torch.mm(a.cuda(), bg)
+    exp = a.double() @ b.double()
+    got = ntops_amd.torch.addmm(c.cuda(), a.cuda(), bg)
+    assert _lib.last_kernel().startswith("gemm_mfma 256x256 s4"), _lib.last_kernel()
     assert _lib.last_kernel().endswith("even+edges"), _lib.last_kernel()
-    exp = (a.double() @ b.double()).float().bfloat16()
-    assert torch.equal(got.cpu(), exp)
-    bias = (0.1 * torch.randn(n, generator=g)).bfloat16()
+    assert torch.equal(got.cpu(), (exp + c.double()).float().bfloat16())
+    got = ntops_amd.torch.mm(a.cuda(), bg)
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
+    assert torch.equal(got.cpu(), exp.float().bfloat16())
+    c = (0.1 * torch.randn(m, cn, generator=g)).bfloat16()
     af, bf_ = (0.1 * torch.randn(m, k, generator=g)).bfloat16(), (0.1 * torch.randn(k, n, generator=g)).bfloat16()
     bfg = bf_.cuda() if not b_kmajor else bf_.t().contiguous().cuda().t()
-    got = ntops_amd.torch.addmm(bias.cuda(), af.cuda(), bfg, beta=0.5, alpha=2.0)
+    got = ntops_amd.torch.addmm(c.cuda(), af.cuda(), bfg, beta=0.5, alpha=2.0)
     rows = tile_rows(m)
-    check(got[rows], af[rows], bf_, torch.bfloat16, c=bias.expand(len(rows), n), alpha=2.0, beta=0.5,
+    check(got[rows], af[rows], bf_, torch.bfloat16, c=c[rows].expand(len(rows), n), alpha=2.0, beta=0.5,
           what="addmm interior + edges")
 
 
-def test_bmm_even_interior_and_edge_strips():
-    """A batch of products whose M and N are not multiples of 256: the
-    interior and both strips of every batch member (the strips offset inside
-    each member, the batch strides unchanged).  Exact small-integer sums."""
+def test_batch_even_interior_and_edge_strips():
+    """A batch of products whose M and N are not multiples of 256, each under
+    its own C: the interior and both strips of every batch member (the strips
+    offset inside each member, the batch strides unchanged).  Exact
+    small-integer sums."""
     g = torch.Generator().manual_seed(23)
     a = torch.randint(-8, 9, (4, 2100, 320), generator=g).to(torch.bfloat16)
     b = torch.randint(-8, 9, (4, 320, 2060), generator=g).to(torch.bfloat16)
-    got = ntops_amd.torch.bmm(a.cuda(), b.cuda())
+    c = torch.randint(-8, 9, (4, 2100, 2060), generator=g).to(torch.bfloat16)
+    exp = torch.bmm(a.double(), b.double())
+    b = torch.nn.functional.pad(b, (0, 4))  # rows of 2064: 16-byte aligned
+    ag, bg, cg = a.cuda(), b.cuda(), c.cuda()
+    out = torch.full(c.shape, float("nan"), dtype=c.dtype, device="cuda")
+    c_gemm(ag, bg.transpose(1, 2).contiguous()[:, :2060].transpose(1, 2), cg, cg.stride(), out, out.stride())
     assert _lib.last_kernel().endswith("even+edges"), _lib.last_kernel()
-    assert torch.equal(got.cpu(), torch.bmm(a.double(), b.double()).float().bfloat16())
+    assert torch.equal(out.cpu(), (exp + c.double()).float().bfloat16())
+    got = ntops_amd.torch.bmm(ag, bg[:, :, :2060])
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
+    assert torch.equal(got.cpu(), exp.float().bfloat16())
 
 
 @pytest.mark.parametrize("m, n, k", [(2048, 16387, 320), (4100, 8195, 512)])
-def test_mm_shifted_rows_exact(m, n, k):
+def test_shifted_rows_exact(m, n, k):
     """Odd N with a K-major B (F.linear's weight): output rows start at every
-    2-byte offset, so the full interior tiles store 16-byte chunks shifted to
-    aligned addresses (plus element stores at each row segment's two ends)
-    and the edge strips store element by element.  Small-integer operands:
-    every output equals the double-precision product rounded once to bf16."""
+    2-byte offset.  Under a C with a value per element the full interior tiles
+    store 16-byte chunks shifted to aligned addresses (plus element stores at
+    each row segment's two ends) and the edge strips store element by element;
+    without a C the persistent kernel stores rows at any offset.  Small-integer
+    operands: every output equals the double-precision result rounded once to
+    bf16."""
     g = torch.Generator().manual_seed(m + n + k)
     a = torch.randint(-8, 9, (m, k), generator=g).to(torch.bfloat16)
     w = torch.randint(-8, 9, (n, k), generator=g).to(torch.bfloat16)
-    got = ntops_amd.torch.mm(a.cuda(), w.cuda().t())
+    c = torch.randint(-8, 9, (m, n), generator=g).to(torch.bfloat16)
+    exp = a.double() @ w.double().t()
+    got = ntops_amd.torch.addmm(c.cuda(), a.cuda(), w.cuda().t())
     assert _lib.last_kernel().endswith("even+edges"), _lib.last_kernel()
-    assert torch.equal(got.cpu(), (a.double() @ w.double().t()).float().bfloat16())
+    assert torch.equal(got.cpu(), (exp + c.double()).float().bfloat16())
+    got = ntops_amd.torch.mm(a.cuda(), w.cuda().t())
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
+    assert torch.equal(got.cpu(), exp.float().bfloat16())
 
 
-def test_gemm_shifted_rows_full_tiles_through_the_c_abi():
-    """A row stride of an odd element count over full 256 x 256 tiles (the
-    even kernel alone) with a bias: shifted 16-byte stores everywhere; the
-    bytes between the rows stay untouched."""
-    lib = _lib.load()
+@pytest.mark.parametrize("form, kernel", (("full", "gemm_mfma 256x256 s4 A:K B:N even"), ("row", "gemm_large A:K B:N")))
+def test_gemm_shifted_rows_full_tiles_through_the_c_abi(form, kernel):
+    """A row stride of an odd element count over full 256 x 256 tiles: with a
+    full C the even kernel alone, its stores shifted 16-byte chunks everywhere;
+    with a bias row the persistent kernel.  The bytes between the rows stay
+    untouched."""
     m, n, k = 4096, 4096, 384
     g = torch.Generator().manual_seed(17)
     a = torch.randint(-8, 9, (m, k), generator=g).to(torch.bfloat16)
     b = torch.randint(-8, 9, (k, n), generator=g).to(torch.bfloat16)
-    bias = torch.randint(-8, 9, (n,), generator=g).to(torch.bfloat16)
+    c = torch.randint(-8, 9, (m if form == "full" else 1, n), generator=g).to(torch.bfloat16)
     big = torch.zeros(m, n + 5, dtype=torch.bfloat16, device="cuda")
     out = big[:, 1:1 + n]
-    ag, bg, biasg = a.cuda(), b.cuda(), bias.cuda()
-    rc = lib.ntops_gemm(_lib.dtype_code(torch.bfloat16), 1, m, n, k, ag.data_ptr(), _lib.i64_array((0, k, 1)),
-                        bg.data_ptr(), _lib.i64_array((0, n, 1)), biasg.data_ptr(), _lib.i64_array((0, 0, 1)),
-                        1.0, 1.0, out.data_ptr(), _lib.i64_array((0, n + 5, 1)), _lib.stream_of(out))
-    _lib.check(rc, "ntops_gemm shifted rows")
-    assert _lib.last_kernel().startswith("gemm_mfma 256x256 s4 A:K B:N even"), _lib.last_kernel()
+    c_gemm(a.cuda()[None], b.cuda()[None], c.cuda(), (0, n if form == "full" else 0, 1), out, (0, n + 5, 1))
+    assert _lib.last_kernel() == kernel, _lib.last_kernel()
     torch.cuda.synchronize()
     assert big[:, 0].abs().sum() == 0 and big[:, 1 + n:].abs().sum() == 0
-    exp = (a.double() @ b.double() + bias.double()).float().bfloat16()
-    assert torch.equal(out.cpu(), exp)
+    assert torch.equal(out.cpu(), (a.double() @ b.double() + c.double()).float().bfloat16())
 
 
 # K not a multiple of 8 (or of 4): A's rows and B's columns zero-extended so
@@ -675,7 +704,9 @@ def test_addmm_c_forms(dtype, form, shape):
         out = torch.empty(m * n + 4, dtype=dtype, device="cuda")[4:].view(m, n)
         assert out.data_ptr() % 16 == 8
     got = ntops_amd.torch.addmm(cg, a.cuda(), b.cuda(), beta=0.75, alpha=1.5, out=out)
-    assert _lib.last_kernel().startswith("gemm_mfma " + shape.split()[0])
+    tile = shape.split()[0]
+    large = tile == "256" and form == "row_bias"  # one row for all: the persistent kernel
+    assert _lib.last_kernel().startswith("gemm_large " if large else f"gemm_mfma {tile}x{tile} "), _lib.last_kernel()
     rows = tile_rows(m) if m > 1024 else None
     assert_gemm_ulp(got, a, b, DT_NAME[dtype], c, 1.5, 0.75, f"addmm C {form} {shape}", rows=rows)
 
@@ -754,7 +785,7 @@ def _config_mm():
     return a, b, bias
 
 
-CONFIG_KERNEL = "gemm_mfma 256x256 s4 A:K B:N even"
+CONFIG_KERNEL = "gemm_large A:K B:N"
 
 
 def test_mm_and_addmm_config_full_size():

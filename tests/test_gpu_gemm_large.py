@@ -40,7 +40,7 @@ def test_large_tiles_exact(m, n, k, layout, dtype):
     exp = a.double() @ b.double()
     ag, bg = major(a, layout[0]), major(b, layout[1])
     got = T.mm(ag, bg)
-    assert _lib.last_kernel().startswith("gemm_mfma 256x256"), _lib.last_kernel()
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
     assert torch.equal(got, exp.float().to(dtype))
     assert torch.equal(T.addmm(bias, ag, bg), (exp + bias.double()).float().to(dtype))
     got = T.addmm(bias, ag, bg, beta=0.5, alpha=2.0)
@@ -62,7 +62,7 @@ def test_large_tiles_output_views(form):
         big = torch.full((m + 2, n + (5 if form == "odd stride" else 8)), 7.0, dtype=dtype, device="cuda")
         out = big[1:1 + m, 3:3 + n]
     T.addmm(torch.zeros(n, dtype=dtype, device="cuda"), a, b, out=out)
-    assert _lib.last_kernel().startswith("gemm_mfma 256x256"), _lib.last_kernel()
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
     assert torch.equal(out, exp)
     kept = big.float().sum() - out.float().sum()
     assert kept.item() == 7.0 * (big.numel() - out.numel())
@@ -75,11 +75,12 @@ def test_large_tiles_batch_and_full_c():
     a, b = ints(5, 2000, 264, seed=6, dtype=dtype), ints(5, 264, 2056, seed=7, dtype=dtype)
     exp = torch.stack([x.double() @ y.double() for x, y in zip(a, b)]).float().to(dtype)
     assert torch.equal(T.bmm(a, b), exp)
-    assert _lib.last_kernel().startswith("gemm_mfma 256x256"), _lib.last_kernel()
+    assert _lib.last_kernel().startswith("gemm_large "), _lib.last_kernel()
     a, b, c = ints(4096, 512, seed=8, dtype=dtype), ints(512, 4096, seed=9, dtype=dtype), ints(4096, 4096, seed=10, dtype=dtype)
     exp = a.double() @ b.double()
-    assert torch.equal(T.addmm(c, a, b), (exp + c.double()).float().to(dtype))
-    assert torch.equal(T.addmm(c[:, :1], a, b), (exp + c[:, :1].double()).float().to(dtype))
+    for cv in (c, c[:, :1]):
+        assert torch.equal(T.addmm(cv, a, b), (exp + cv.double()).float().to(dtype))
+        assert _lib.last_kernel() == "gemm_mfma 256x256 s4 A:K B:N even", _lib.last_kernel()
 
 
 @pytest.mark.parametrize("m, n, k, layout, large", (
@@ -105,6 +106,6 @@ def test_large_tiles_below_a_round(m, n, k, layout, large):
     ag, bg = major(a, layout[0]), major(b, layout[1])
     got = T.mm(ag, bg)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
-        assert _lib.last_kernel().startswith("gemm_mfma 256x256" if large else "gemm_mfma 128x128"), _lib.last_kernel()
+        assert _lib.last_kernel().startswith("gemm_large " if large else "gemm_mfma 128x128"), _lib.last_kernel()
     assert torch.equal(got, exp.float().to(dtype))
     assert torch.equal(T.addmm(bias, ag, bg), (exp + bias.double()).float().to(dtype))
