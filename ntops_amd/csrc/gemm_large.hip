@@ -655,23 +655,26 @@ int gemm_large(int dtype, bool a_kmajor, bool b_kmajor, const GemmArgs& g, hipSt
 // the count where 128 x 128 tiles (two to a CU) need a second round on they
 // are still faster: bf16 K-major B, 2560 x 4096 x 4096 (160 tiles) 106.9 -> 70.2
 // us, 3584 x 4096 x 4096 (224) 145.7 -> 84.1, 2816 x 3072 x 768 (132) 25.0 ->
-// 20.1, 2816 x 3072 x 512 19.4 -> 16.5, N-major within 4 %.  Products whose
-// last row or column of large tiles is half empty or more take it from K = 2048
-// on (257 x 25600 x 4096 121.2 -> 73.7, 2050 x 4096 x 2048 68.0 -> 39.9); shorter
-// ones would gain too (2050 x 4096 x 1024 38.7 / 26.6) but keep the kernel that
-// test_gpu_gemm.py states for them.  Where the small tiles fill seven eighths of
-// their one round, a K of k_min or more amortises the large kernel's fill: 2048 x
-// 4096 x 4096 (128) 80.0 -> 65.8, but 3584 x 2304 x 768 (126) 19.1 -> 20.0; not
-// with half empty large tiles (a product of 128 rows).  Below that the small
-// ones are as fast or faster (768 x 6400 x 1600, 75: 34.0 / 32.2; 1024 x 4096 x
-// 4096, 64: 38.7 / 64.5).
+// 20.1, 2816 x 3072 x 512 19.4 -> 16.5, N-major within 4 %.  That holds where
+// the last row or column of large tiles is half empty or more, too (small ->
+// large, K-major B / N-major B): 2050 x 4096 x 512 23.1 -> 16.8 / 23.3 -> 17.5, x
+// 1024 37.4 -> 23.3 / 37.5 -> 24.2, x 2040 78.7 -> 43.3 / 68.2 -> 40.6; the
+// least, half empty tiles at K = 512, 1152 x 8192 19.2 -> 17.1 / 18.3 -> 18.0
+// (M-major A: 20.0 -> 18.2 / 18.9 -> 19.0); convolutions 3 x 3 of 64 channels (40,
+// 28 x 28) to 256 37.8 -> 32.3, 1 x 1 of 512 52.8 -> 46.4.  Below K = 512 an
+// N-major B starts to lose (x 448: 2560 x 4096 16.8 -> 17.4, 1152 x 8192 17.1 ->
+// 18.1), a K-major one still gains (17.6 -> 16.5, 18.0 -> 17.1).  Where the
+// small tiles fill seven eighths of their one round, a K of k_min or more
+// amortises the large kernel's fill: 2048 x 4096 x 4096 (128) 80.0 -> 65.8, but
+// 3584 x 2304 x 768 (126) 19.1 -> 20.0; not with half empty large tiles (a product
+// of 128 rows).  Below that the small ones are as fast or faster (768 x 6400 x
+// 1600, 75: 34.0 / 32.2; 1024 x 4096 x 4096, 64: 38.7 / 64.5).
 bool large_tiles_suit(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t k_min) {
   const int64_t cus = cu_count_cached() > 0 ? cu_count_cached() : 256;
   const int64_t large = ((M + 255) / 256) * ((N + 255) / 256) * batch;
   const int64_t small = ((M + 127) / 128) * ((N + 127) / 128) * batch;
   const bool whole = small == 4 * large;
-  return large >= 240 || (small > 2 * cus && K >= (whole ? 512 : 2048)) ||
-         (whole && 4 * small > 7 * cus && K >= k_min);
+  return large >= 240 || (small > 2 * cus && K >= 512) || (whole && 4 * small > 7 * cus && K >= k_min);
 }
 
 // Where the plain kernel's tiles suit (K > 256), on images whose

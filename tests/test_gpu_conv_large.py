@@ -24,12 +24,13 @@ def small_ints(g, *shape):
     return torch.randint(-2, 3, shape, generator=g).float()
 
 
-# (n, c, h, w, k, (r, s), stride, padding, dilation, bias): each reaches 240 tiles
+# (n, c, h, w, k, (r, s), stride, padding, dilation, bias): each reaches 240 tiles, or 512 small ones
 CASES = [
     (240, 64, 16, 16, 256, (3, 3), 1, 1, 1, True),     # even; 9 K tiles (the last pair half empty)
     (128, 320, 18, 18, 256, (1, 1), 1, 0, 1, False),   # 1 x 1: 5 K tiles, the fewest; 324 pixels: two tiles an image
     (62, 64, 64, 48, 130, (3, 3), (2, 1), (1, 1), 1, True),  # ragged rows, stride 2 down, 1536 pixels
     (2, 64, 180, 180, 256, (3, 5), 1, (2, 4), 2, True),      # many pixels, unequal taps, dilation
+    (40, 64, 28, 28, 256, (3, 3), 1, 1, 1, True),      # 160 tiles, the last of each image 16 pixels
     (128, 128, 20, 17, 256, (5, 1), 1, (2, 0), 1, False),    # element copy of the input (rows not 16 bytes)
 ]
 

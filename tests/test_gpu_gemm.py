@@ -74,7 +74,13 @@ def expected16(m, n, k, layout, batch=1):
         return "gemm_skinny "
     if k <= 128 and m % 128 == 0 and n % 128 == 0:
         return "gemm_panel "
-    if -(-m // 256) * -(-n // 256) * batch >= 240 and k > 256:
+    # the persistent kernel: a round of 256 x 256 tiles, or what takes the 128 x
+    # 128 ones (two to a CU) past their one round or, where no 256 x 256 tile is
+    # half empty, to seven eighths of it
+    large = -(-m // 256) * -(-n // 256) * batch
+    k_min = 1024 if b_k else 2048
+    if k > 256 and (large >= 240 or (tiles > 2 * cus and k >= 512)
+                    or (a_k and tiles == 4 * large and 4 * tiles > 7 * cus and k >= k_min)):
         return "gemm_large "
     return "gemm_mfma 128x128 "
 

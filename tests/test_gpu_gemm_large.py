@@ -88,8 +88,10 @@ def test_large_tiles_batch_and_full_c():
     (2553, 3321, 512, "NT", True),     # the same, ragged
     (2560, 3328, 520, "TN", True),
     (2560, 3328, 504, "NT", False),    # too short for it
-    (2050, 4096, 2048, "NT", True),    # 544, the last row of large tiles nearly empty
-    (2050, 4096, 2040, "NN", False),
+    (2050, 4096, 512, "NT", True),     # 544, the last row of large tiles nearly empty
+    (2050, 4096, 1024, "NN", True),
+    (1152, 8192, 520, "TN", True),     # 576, the last row of large tiles half empty
+    (2050, 4096, 504, "NN", False),
     (2048, 4096, 1024, "NT", True),    # 512: one full round, K-major B
     (2048, 4096, 1016, "NT", False),
     (2048, 4096, 2048, "NN", True),    # N-major B from K = 2048
