@@ -38,6 +38,7 @@
 // 64.8, (32, 64, 112, 112) to 128 152.8 -> 136.2.  What is left there is the
 // input's copy (19 us) and 416 tiles over 256 CUs: two rounds, 0.8 full.
 #include <algorithm>
+#include <atomic>
 
 #include "gemm.h"
 #include "gemm_tile.h"
@@ -60,8 +61,6 @@ __device__ __forceinline__ int here(int lane) {
   return lane;
 }
 
-// This lane's fragment reads of one operand: a 32-row (or column) slice of a
-// half tile, 16 k per read.
 // v_mfma_f32_16x16x32: lane l holds row / column l & 15 at k = 8 (l >> 4) ..
 // + 7 of A / B; of the result column l & 15 and rows 4 (l >> 4) .. + 3.
 template <typename T>
@@ -74,7 +73,8 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                   0);
 }
 
-// TILES slices of 16 rows, 32 k per read.
+// This lane's fragment reads of one operand: TILES slices of 16 rows (or
+// columns) of a half tile, 32 k per read.
 template <bool KMAJ, int TILES>
 struct FragReader {
   // LDS byte addresses at half 0 of buffer 0: per k-step, or per two slices
@@ -305,8 +305,9 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
       lb.template issue<decltype(tail)::value>(rs.b[half], lds, t * 64, g.K, wave, lane);
   };
 
-  f32x4 acc[4][2][4];  // [quadrant][row tile][column tile]
-  //  // quadrants 00, 10, 11, 01 (row half, column half), 32 x 64 per wave
+  // [quadrant][row tile][column tile]; quadrants 00, 10, 11, 01 (row half,
+  // column half), 32 x 64 per wave
+  f32x4 acc[4][2][4];
   u32x4 ax[4], ay[4], bx[4][2];  // A0, A1, one half of B
   FragReader<AK, 2> fa;
   FragReader<BKM, 4> fb;
@@ -603,12 +604,12 @@ __global__ __launch_bounds__(512, 1) void k_gemm_large(GemmArgs g, int total) {
 template <typename T, bool AK, bool BKM, bool BIAS, bool CONV = false>
 int launch_large(const GemmArgs& g, hipStream_t st) {
   auto kern = k_gemm_large<T, AK, BKM, BIAS, CONV>;
-  static bool attr_set = false;
-  if (!attr_set) {
+  static std::atomic<bool> attr_set{false};  // (threads may get here together)
+  if (!attr_set.load(std::memory_order_relaxed)) {
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             kLargeLds) != hipSuccess)
       return set_error(NTOPS_ERR_HIP, "gemm: cannot reserve %d bytes of LDS", kLargeLds);
-    attr_set = true;
+    attr_set.store(true, std::memory_order_relaxed);
   }
   const int64_t total = static_cast<int64_t>((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
   if (total > 0x3fffffffLL) return set_error(NTOPS_ERR_UNSUPPORTED, "gemm: too many tiles");
