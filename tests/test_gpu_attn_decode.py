@@ -65,6 +65,24 @@ def test_decode(b, hq, hkv, sq, skv, d, causal, dtype):
     assert_close(out, oracle(q, k, v, causal), 1.6e-2, 1.6e-2, "unsplit")
 
 
+# a key / value head for every CU: any cache is served, of one key up to a tile
+# and past it, and rows that see no key at all (lower-right, fewer keys than
+# queries) are zero
+@pytest.mark.parametrize("sq, skv, causal", ((1, 1, 0), (1, 7, 0), (1, 31, 0), (2, 33, 1), (1, 64, 0), (4, 65, 2),
+                                             (1, 256, 0), (16, 5, 2), (16, 1, 2), (3, 40, 1)))
+@pytest.mark.parametrize("d", (64, 128))
+def test_decode_short_caches(sq, skv, causal, d):
+    b, h = (16, 16) if torch.cuda.get_device_properties(0).multi_processor_count <= 256 else (32, 32)
+    g = torch.Generator().manual_seed(skv + d)
+    q, k, v = (torch.randn(b, h, s, d, generator=g).bfloat16() for s in (sq, skv, skv))
+    got = sdpa(q.cuda(), k.cuda(), v.cuda(), is_causal=causal > 0,
+               causal_variant=CausalVariant(causal) if causal else None)
+    assert _lib.last_kernel().startswith("sdpa_decode"), _lib.last_kernel()
+    assert_close(got, oracle(q, k, v, causal), 1.6e-2, 1.6e-2, "short cache")
+    if causal == 2 and sq > skv:
+        assert (got[:, :, :sq - skv] == 0).all()
+
+
 @pytest.mark.parametrize("b, h", ((1, 2), (8, 32)))
 @pytest.mark.parametrize("causal", (0, 2))
 def test_empty_cache(b, h, causal, monkeypatch):
@@ -87,7 +105,7 @@ def test_empty_cache(b, h, causal, monkeypatch):
 
 
 def test_decode_special_values():
-    """NaN and infinite scores, a causal row that sees no key, and a repeated
+    """NaN and infinite scores, a causal row that sees one key, and a repeated
     call (bit for bit: the slices are combined in a fixed order)."""
     q = torch.randn(1, 4, 1, 64, device="cuda").bfloat16()
     k, v = (torch.randn(1, 2, 900, 64, device="cuda").bfloat16() for _ in range(2))
@@ -102,7 +120,7 @@ def test_decode_special_values():
     k2[:, 0, :, 5] = float("-inf")
     q[0, :, 0, 5] = 1.0
     assert (sdpa(q, k2, v, enable_gqa=True)[0, :2] == 0).all()
-    # lower-right with more queries than keys: the first rows see no key
+    # upper-left: the first row sees the first key alone
     q = torch.randn(1, 1, 16, 64, device="cuda").half()
     k, v = (torch.randn(1, 1, 300, 64, device="cuda").half() for _ in range(2))
     got = sdpa(q, k, v, is_causal=True)

@@ -2,6 +2,7 @@
 bit for bit over the forms each op accepts, the same errors for those it
 refuses, and None (the Python path) for tensors that are not plain."""
 
+import collections
 import ctypes
 import itertools
 from concurrent.futures import ThreadPoolExecutor
@@ -63,9 +64,12 @@ def forms():
                                                 ("NN", "NT", "TN")):
             a = u(m, k) if lay[0] == "N" else u(k, m).t()
             b = u(k, n) if lay[1] == "N" else u(n, k).t()
-            yield "mm", lambda a=a, b=b: T.mm(a, b)
-            for c in (u(n), u(m, n), u(m, 1), u(1, n), u(1), u(n, m).t(), u(n + 1)):
-                yield "addmm", lambda a=a, b=b, c=c: T.addmm(c, a, b, beta=0.5, alpha=2)
+            # (K-major rows of whole 16-byte runs are what the native path takes)
+            kind = "mm odd k" if k % (4 if dtype == torch.float32 else 8) else "mm " + lay
+            yield kind, lambda a=a, b=b: T.mm(a, b)
+            for cname, c in (("row", u(n)), ("full", u(m, n)), ("column", u(m, 1)), ("row", u(1, n)), ("scalar", u(1)),
+                             ("transposed", u(n, m).t()), ("mismatch", u(n + 1))):
+                yield "addmm " + cname, lambda a=a, b=b, c=c: T.addmm(c, a, b, beta=0.5, alpha=2)
         yield "mm mismatch", lambda: T.mm(u(4, 16), u(24, 32))
         yield "mm dtypes", lambda: T.mm(u(4, 16), u(16, 32).double())
         for hq, hk, d in ((4, 4, 64), (4, 2, 128), (3, 3, 20)):
@@ -74,8 +78,9 @@ def forms():
             yield "sdpa causal", lambda q=q, k=k, v=v: T.scaled_dot_product_attention(
                 q.transpose(1, 2).contiguous().transpose(1, 2), k, v, is_causal=True, enable_gqa=True, scale=0.3,
                 causal_variant=2)
-            for m in (r(5, 300) > 0, u(2, 1, 1, 300), r(2, hq, 5, 300, dtype=torch.float32), r(4, 300) > 0):
-                yield "sdpa mask", lambda q=q, k=k, v=v, m=m: T.scaled_dot_product_attention(
+            for mname, m in (("bool", r(5, 300) > 0), ("own dtype", u(2, 1, 1, 300)),
+                             ("f32", r(2, hq, 5, 300, dtype=torch.float32)), ("mismatch", r(4, 300) > 0)):
+                yield "sdpa mask " + mname, lambda q=q, k=k, v=v, m=m: T.scaled_dot_product_attention(
                     q, k, v, attn_mask=m, enable_gqa=True)
             yield "sdpa heads", lambda q=q, k=k, v=v: T.scaled_dot_product_attention(q[:, :1], k, v)
             yield "sdpa 3-D", lambda q=q, k=k, v=v: T.scaled_dot_product_attention(q[0], k[0], v[0], enable_gqa=True)
@@ -90,8 +95,8 @@ def forms():
         for d, tw in ((64, 64), (64, 32), (24, 24)):
             q, k, s, c = u(2, 9, 4, d), u(2, 9, 2, d), u(9, tw), u(11, tw)
             for inter in (False, True):
-                yield "rope", lambda q=q, k=k, s=s, c=c, i=inter: T.rotary_position_embedding_qk(q, k, s, c, i)
-            yield "rope f32 tables", lambda q=q, k=k, s=s, c=c: T.rotary_position_embedding_qk(
+                yield "rope " + ("interleaved" if inter else "half"), lambda q=q, k=k, s=s, c=c, i=inter: T.rotary_position_embedding_qk(q, k, s, c, i)
+            yield "rope f32 tables" if dtype != torch.float32 else "rope half", lambda q=q, k=k, s=s, c=c: T.rotary_position_embedding_qk(
                 q.transpose(0, 1), k.transpose(0, 1), s.float(), c.float(), False)
 
 
@@ -107,16 +112,34 @@ def outcome(call):
 @pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
 def test_native_and_python_paths_agree(monkeypatch):
     assert _lib.fast is not None, "the extension is not built"
-    served = 0
+    served, native = 0, collections.Counter()
+
+    class Counting:
+        """The extension, counting per form and function the calls it serves."""
+
+        def __getattr__(self, fn):
+            def call(*args):
+                r = getattr(fast, fn)(*args)
+                if r is not None:
+                    hits.append(fn)
+                    native[name] += 1
+                    native["fast." + fn] += 1
+                return r
+            return call
+
+    fast = _lib.fast
     for name, call in forms():
-        got = outcome(call)
-        fast = _lib.fast
+        hits = []
+        with monkeypatch.context() as mp:
+            mp.setattr(_lib, "fast", Counting())
+            got = outcome(call)
         with monkeypatch.context() as mp:
             mp.setattr(_lib, "fast", None)
             exp = outcome(call)
         assert _lib.fast is fast
         if isinstance(exp[0], type):
             assert got == exp, (name, got, exp)
+            assert not hits, (name, "refused in Python, served natively")
             continue
         assert not isinstance(got[0], type), (name, got)
         served += 1
@@ -124,13 +147,16 @@ def test_native_and_python_paths_agree(monkeypatch):
             assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride(), name
             assert torch.equal(a, b) or (torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())), name
     assert served > 300
-    # the usual forms are served natively
-    x = torch.randn(4, 64, device="cuda").bfloat16()
-    w = torch.randn(64, device="cuda").bfloat16()
-    assert _lib.fast.add_rms_norm(x, x, (64,), w, 1e-6) is not None
-    assert _lib.fast.mm(x, torch.randn(32, 64, device="cuda").bfloat16().t()) is not None
-    q = torch.randn(1, 2, 4, 64, device="cuda").half()
-    assert _lib.fast.sdpa(q, q, q, None, 1, None, False, None, None, None, None) is not None
+    # every function and every form that is meant to be served natively was
+    for fn in ("unary", "softmax", "rms_norm", "layer_norm", "add_rms_norm", "rope_qk", "mm", "addmm", "sdpa"):
+        assert native["fast." + fn], fn
+    for form in ("silu", "gelu", "norm of two dims", "rms_norm int", "mm NN", "mm NT", "addmm row", "addmm full",
+                 "addmm column", "addmm transposed", "sdpa", "sdpa causal", "sdpa mask bool", "sdpa mask own dtype",
+                 "sdpa mask f32", "sdpa cache", "rope interleaved", "rope half"):
+        assert native[form], form
+    # and the others were left to Python
+    for form in ("mm TN", "mm odd k", "sdpa 3-D", "rope f32 tables"):
+        assert not native[form], form
     # on another stream the work is ordered on that stream
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
