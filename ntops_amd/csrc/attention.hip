@@ -62,6 +62,16 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 
+// a * b rounded down.
+__device__ __forceinline__ float mul_down(float a, float b) {
+  const float u = mul_nc(a, b);
+  return fmaf(a, b, -u) < 0.f ? fmaf(fabsf(u), -0x1.8p-24f, u) : u;  // u less its last place
+}
+
+// From here on a result cut to [0, 1] keeps a NaN (it is 0 by default): the
+// wave's MODE register, bit 8 (DX10_CLAMP).
+__device__ __forceinline__ void clamp_keeps_nan() { __builtin_amdgcn_s_setreg(1 | 8 << 6 | 0 << 11, 0); }
+
 // Max of a lane's 32 scores of a tile: 16 three-way maxima in a tree.
 __device__ __forceinline__ float max32(const f32x16 (&s)[2]) {
   float v[32];
@@ -196,9 +206,9 @@ __device__ __forceinline__ u32x4 times_zero(u32x4 x) {
 }
 
 // MM: explicit-mask mode -- 0 none, 1 / 2 the last, partial tile by runs of 4
-// keys (rows 4-element aligned) / by elements; ESZ: mask element bytes (1 bool, 2
-// fp16 / bf16, 4 fp32).  Both are template parameters so that every mask
-// load writes fixed registers.
+// keys (rows 4-element aligned) / by elements; ESZ: mask element bytes (1 bool,
+// 2 fp16 / bf16, 4 fp32; without a mask 0 for a zero scale, 1 for any other).
+// Both are template parameters so that every mask load writes fixed registers.
 template <typename T, int D, int MM, int ESZ>
 __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int total) {
   constexpr int BM = 128, BN = 64;
@@ -213,6 +223,7 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
   const int wave = threadIdx.x >> 6;
   int bh, qb;
   if (block_id() >= total) return;  // the tail of a 2-D grid (the whole block)
+  clamp_keeps_nan();
   attn_block(static_cast<int>(block_id()), total, nqb, bh, qb);
   const int b = bh / a.Hq, h = bh - b * a.Hq;
   const int hk = h / (a.Hq / a.Hkv);
@@ -235,11 +246,12 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       qf[ks] = u32x4{0, 0, 0, 0};
   }
   // a negative scale: -Q under its magnitude, so that the max of the scaled
-  // scores is the scaled max; a zero scale (MM = 0 only): 0 Q under one, so
-  // that a key without a score stays at -inf
+  // scores is the scaled max; a zero scale: 0 Q under one, so that a key
+  // without a score stays at -inf (an instantiation of its own: the selects
+  // took 2 % of the others' time)
+  constexpr bool zero = ESZ == 0;
   const bool neg = a.scale_log2 < 0.f;
-  const bool zero = a.scale_log2 == 0.f;
-  if (zero) {
+  if constexpr (zero) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = times_zero<T>(qf[ks]);
   }
@@ -432,14 +444,6 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
   float m_i = neg_inf(), l_i = 0.f;  // reference max (base 2) of row my_q; this lane's half of its sum
   const float c = zero ? 1.f : neg ? -a.scale_log2 : a.scale_log2;
-  // m_i is the rounded product max(S) c, which the fma's exact one misses by
-  // up to half an ulp: nothing near zero (2^-15 of P's exponent at 2^10), but
-  // 64 at the 1e10 of a row that a large finite mask value closes, which took
-  // P to 0 or past f16.  From kFarMax on the scores are rounded like m_i, so
-  // that the largest P is exactly 1.  ((8, 16, 1000, 64) f16 bool 60.8 us
-  // without the test, 61.2 with it.)
-  constexpr float kFarMax = 1024.f;
-  bool far = false;  // some row of the wave is there
   // last key of row my_q, relative to this lane's column group
   int lim = a.Skv - 1;
   if (a.causal) lim = min(lim, my_q + off);
@@ -505,10 +509,19 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
     // rescaled, and the halves exchange their maxima, only on tiles that raise
     // some row's max.  (The max itself stays the reference: a row's largest P
     // is then 1 and carries no rounding, where a reference raised only past
-    // 2^8 of it, as in k_flash_attn, is 2.5 % further from 64 bits.)
-    const float th = max32(s) * c;
+    // 2^8 of it, as in k_flash_attn, is 2.5 % further from 64 bits.)  The fma's
+    // product is exact; a reference rounded to nearest is up to half a unit of
+    // its last place off: nothing for scores near zero, but 64 at the 1e10 of a
+    // row that a large finite mask value closes, which took P to 0 or past f16.
+    // Rounded down, it leaves no largest exponent negative, and P is cut at 1 (a
+    // result modifier of the exponential, no instruction).  (1, 32, 128, 64) over
+    // 700 keys: 13.2 us with the halves' maxima exchanged through the LDS, 12.6 by
+    // a swap of registers; 12.9 with neither, 13.5 where a vote per tile found
+    // such references and rounded the scores too.
+    const float th = mul_down(max32(s), c);
     if (__any(th > m_i)) {
-      const float tmax = fmaxf(th, __shfl_xor(th, 32, 64));
+      const auto h2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(th), __float_as_uint(th), false, false);
+      const float tmax = fmaxf(__uint_as_float(h2[0]), __uint_as_float(h2[1]));  // of lanes l and l ^ 32
       const bool up = tmax > m_i;
       const float alpha = up ? fast_exp2(m_i - tmax) : 1.f;
       m_i = up ? tmax : m_i;
@@ -517,21 +530,13 @@ __global__ __launch_bounds__(256, 2) void k_flash_fwd(AttnArgs a, int nqb, int t
       for (int t = 0; t < DT; ++t)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
-      far = __any(fabsf(m_i) >= kFarMax && m_i > neg_inf());
     }
     const float mb = m_i == neg_inf() ? 0.f : m_i;  // fully masked so far: P = 0
     float x[2][16];
-    if (far) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(add_nc(mul_nc(s[t][e], c), -mb));
-    } else {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[t][e] = fast_exp2(fmaf(s[t][e], c, -mb));
-    }
+      for (int e = 0; e < 16; ++e) x[t][e] = __builtin_amdgcn_fmed3f(fast_exp2(fmaf(s[t][e], c, -mb)), 0.f, 1.f);
     {
       float r[16];
 #pragma unroll
@@ -1329,7 +1334,8 @@ int run_attention(const AttnArgs& a, void* ws, int64_t ws_bytes, hipStream_t st)
       note_kernel("sdpa_fwd d%d mask%d es%d", a.D > 64 ? 128 : 64, mm, esz);
 #define NTOPS_FWD(DD, MM, ES) hipLaunchKernelGGL((k_flash_fwd<T, DD, MM, ES>), grid, block, 0, st, a, nqb, static_cast<int>(total))
 #define NTOPS_FWD_D(DD)                         \
-  if (mm == 0) NTOPS_FWD(DD, 0, 1);             \
+  if (mm == 0 && a.scale_log2 == 0.f) NTOPS_FWD(DD, 0, 0); \
+  else if (mm == 0) NTOPS_FWD(DD, 0, 1);        \
   else if (mm == 1 && esz == 1) NTOPS_FWD(DD, 1, 1); \
   else if (mm == 1 && esz == 2) NTOPS_FWD(DD, 1, 2); \
   else if (mm == 1) NTOPS_FWD(DD, 1, 4);        \
