@@ -9,6 +9,7 @@ from concurrent.futures import ThreadPoolExecutor
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import ntops_amd
 from ntops_amd import _lib
@@ -218,3 +219,27 @@ def test_native_calls_from_several_threads():
 
     with ThreadPoolExecutor(4) as pool:
         assert all(pool.map(work, range(4)))
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_native_calls_under_a_dispatch_mode():
+    """A mode written in Python sees the native path's allocations, which are
+    made without the interpreter, as it sees the Python path's."""
+    seen = []
+
+    class Seeing(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    x, w = torch.randn(4, 4096, device="cuda").bfloat16(), torch.randn(64, 4096, device="cuda").bfloat16()
+    q, kv = torch.randn(1, 8, 1, 64, device="cuda").half(), torch.randn(1, 2, 2048, 64, device="cuda").half()
+    calls = (lambda: T.silu(x), lambda: T.rms_norm(x, (4096,)), lambda: T.mm(x, w.t()),
+             lambda: T.scaled_dot_product_attention(q, kv, kv, enable_gqa=True))
+    for call in calls:
+        exp = call()
+        seen.clear()
+        with Seeing():
+            got = call()
+        assert seen and torch.equal(got, exp)
