@@ -264,11 +264,11 @@ KERNEL_OF = {
     "rope": "k_rope_half_vec",
     "rope_qk": "k_rope_half_vec",
     "add_rms_norm": "k_add_rms_vec",
-    "mm": "k_gemm_mfma",
-    "addmm": "k_gemm_mfma",
+    "mm": "k_gemm_large",
+    "addmm": "k_gemm_large",
     "bmm": "k_gemm_panel",
     "sdpa": "k_flash_attn",
-    "conv2d": "k_gemm_mfma",
+    "conv2d": "k_gemm_large",
 }
 
 
