@@ -70,8 +70,8 @@ def test_scale_signs(scale, masked):
 
 
 # the large finite values that programs close keys with; tiles of 64 keys
-@pytest.mark.parametrize("value", (-65504.0, -1e6, -1e9, -1e10, -1e30))
-@pytest.mark.parametrize("mask_dtype", (torch.float16, torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("value, mask_dtype", [(-65504.0, torch.float16)] + [
+    (value, dt) for value in (-65504.0, -1e6, -1e9, -1e10, -1e30) for dt in (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize("d", (64, 80, 128))
 def test_large_finite_mask_values(value, mask_dtype, dtype, d):
@@ -81,8 +81,6 @@ def test_large_finite_mask_values(value, mask_dtype, dtype, d):
     they are equal, so the row is the mean of V; with any other the values are
     too coarse for the scores (half a unit and more from 1e6 on), but P still
     sums to 1 and the row lies among V's."""
-    if mask_dtype == torch.float16 and value < -65504:
-        pytest.skip("not a finite value of the type")
     g = torch.Generator().manual_seed(d)
     b, h, sq, skv = 2, 2, 72, 200
     q, k, v = (torch.randn(b, h, s, d, generator=g).to(dtype) for s in (sq, skv, skv))
